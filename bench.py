@@ -179,7 +179,7 @@ def _cpu_model():
 # kernel classes by the kernel each launch runs on the 128^3 operator (the
 # FP32 streaming sweep; Jacobi sweeps and products on the diagonal form)
 SWEEP_KERNEL = "parilu_stream4_sweep_kernel<float>"
-JACOBI_KERNEL = "tri_jacobi_dia_vec_kernel<float>"
+JACOBI_KERNEL = "tri_jacobi_tile_kernel<float>"
 SPMV64_KERNEL = "spmv_dia_kernel<double, float, double>"
 SPMV32_KERNEL = "spmv_dia_kernel<float, float, float>"
 # kernel class -> per-launch timing regions of the library; each launch
@@ -256,9 +256,9 @@ def cache_rates(L, H, n, flush, reps=10):
     cdst = L.DevVec(COPY_BYTES // 8, np.float64)
     cases = [
         (SWEEP_KERNEL, ["parilu_sweep"], lambda: Ps.sweeps(1)),
-        # Jacobi-2: one timed off-diagonal sweep each for L and U
+        # Jacobi-5: one launch of four coupled sweeps each for L and U
         (JACOBI_KERNEL, ["trsv_jacobi_sweep_lower", "trsv_jacobi_sweep_upper"],
-         lambda: L.check(lib.lace_parilu_apply(Pj.h, L.TRSV_JACOBI, 2, 0, r.ptr, z.ptr))),
+         lambda: L.check(lib.lace_parilu_apply(Pj.h, L.TRSV_JACOBI, 5, 0, r.ptr, z.ptr))),
         # FP64 A, x and y (the solve's outer SpMV reads an FP32 x)
         (SPMV64_KERNEL, ["spmv"], lambda: L.check(lib.lace_csr_spmv(A64.h, 1.0, x64.ptr, 0.0, y64.ptr))),
         (SPMV32_KERNEL, ["spmv_f32a"], lambda: L.check(lib.lace_csr_spmv(A32.h, 1.0, x32.ptr, 0.0, y32.ptr))),

@@ -94,6 +94,10 @@ struct TriPlan {
   // which every change of the factor values passes through); tsol is the
   // solution in box order.
   int tile_dims[3] = {0, 0, 0};  // box sides; 0: no box order
+  // The grid's sides when, besides, the diagonal form applies and every row
+  // has an entry for each of its neighbours inside the grid (0: otherwise):
+  // the Jacobi sweeps then run several to a launch on boxes of the grid.
+  int grid[3] = {0, 0, 0};
   DevBuf tperm, trow, tcol, tmap;
   mutable DevBuf tval, tsol;
   mutable const void* tval_src = nullptr;

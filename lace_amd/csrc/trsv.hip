@@ -21,6 +21,7 @@
 #include "common.hpp"
 #include "device.hpp"
 #include "parilu.hpp"
+#include "trsv_tile.hpp"
 
 namespace lace {
 
@@ -131,9 +132,13 @@ static bool tri_grid(int n, const int* row, const int* col, bool upper, long dim
 
 int TriPlan::build_tiles(const int* row_, const int* col_) {
   tile_dims[0] = tile_dims[1] = tile_dims[2] = 0;
+  grid[0] = grid[1] = grid[2] = 0;
   tval_src = nullptr;
   long g[3];
   if (n < 2 || !tri_grid(n, row_, col_, upper, g)) return DEV_SUCCESS;
+  const long full = (g[0] - 1) * g[1] * g[2] + g[0] * (g[1] - 1) * g[2] + g[0] * g[1] * (g[2] - 1);
+  if (dia.nd == (g[2] > 1 ? 3 : 2) && snnz == full)
+    for (int d = 0; d < 3; d++) grid[d] = (int)g[d];
   // 512 rows per box: 8 x 8 x 8 in 3-D, 32 x 16 in 2-D (sides clipped to
   // the grid)
   const long want[3] = {g[2] > 1 ? 8 : 32, g[2] > 1 ? 8 : 16, 8};
@@ -1624,6 +1629,18 @@ int tri_solve_jacobi(const TriPlan& P, const T* val, const T* r, T* y, T* tmp, i
   if (epi_done) *epi_done = false;
   if (sweeps <= 0) {
     LACE_HIP(hipMemsetAsync(y, 0, sizeof(T) * P.n, stream()));
+    return DEV_SUCCESS;
+  }
+  if (r != y && r != tmp && jacobi_tile_ready<T>(P, val, sweeps)) {
+    // boxes of the grid, up to kTileC coupled sweeps a launch in launches of
+    // equal length, ping-ponging so that the last one lands in y
+    const int coupled = sweeps - 1, launches = ceil_div(coupled, kTileC);
+    const T* yin = nullptr;
+    for (int l = 0; l < launches; l++) {
+      T* out = (launches - 1 - l) % 2 == 0 ? y : tmp;
+      LACE_TRY(jacobi_tile<T>(P, r, yin, out, coupled * (l + 1) / launches - coupled * l / launches));
+      yin = out;
+    }
     return DEV_SUCCESS;
   }
   if (P.unit_diag) {
