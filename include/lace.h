@@ -706,7 +706,11 @@ int lace_block_panel_qr(int n, int r0, const double *W, double *Y, double *Tb, d
  * each axis (7- and 5-point stencils, recognised from the pattern alone),
  * the persistent kernel's blocks are boxes of the grid (8 x 8 x 8, or
  * 32 x 16 in 2-D) taken in order of their diagonal (0: blocks of
- * consecutive rows).  Either way the result is bit-identical.
+ * consecutive rows).  "trsv_exact_ring" (0..2, default 1): factors of up
+ * to about 260000 rows whose levels are narrow run in level order on one
+ * workgroup, the last rows of the solution in LDS, where that is expected
+ * to be faster (and "trsv_exact_tiles" and "trsv_exact_rows" are at their
+ * defaults; 2: wherever the form exists).  Either way the result is bit-identical.
  * "inner_ortho" (0 or 1, default 1): the inner GMRES of a nested solve
  * (inner_iters > 0) orthogonalises by classical Gram-Schmidt on an
  * unnormalised basis (1: two vector passes and one small launch per step)

@@ -659,7 +659,7 @@ static void scalar_row_scales(int n, const int* row, const double* val, std::vec
   }
 }
 
-static int build_pattern(const data_d_matrix* A, ParILU* P) {
+static int build_pattern(const data_d_matrix* A, ParILU* P, ParILUUse use) {
   const int n = A->num_rows;
   LACE_REQUIRE(A->num_rows == A->num_cols, DEV_ERR_ILLEGAL_VALUE, "ParILU needs a square matrix");
   LACE_REQUIRE(A->row && A->col && A->val, DEV_ERR_INVALID_PTR, "ParILU: A has null arrays");
@@ -712,6 +712,12 @@ static int build_pattern(const data_d_matrix* A, ParILU* P) {
         dst[k] = -1 - p;
       }
     }
+  const size_t es = P->elem_size();
+  if (!use.sweeps) {
+    // given factors: nothing of A and no second pair of buffers
+    LACE_TRY(P->lval[0].alloc(es * P->nnzL));
+    return P->uval[0].alloc(es * P->nnzU);
+  }
   std::vector<int> rowidx(nnz);
   for (int i = 0; i < n; i++)
     for (int k = A->row[i]; k < A->row[i + 1]; k++) rowidx[k] = i;
@@ -806,7 +812,6 @@ static int build_pattern(const data_d_matrix* A, ParILU* P) {
   // A values in the iteration precision
   DevBuf a64;
   LACE_TRY(upload(a64, A->val, sizeof(double) * nnz));
-  const size_t es = P->elem_size();
   LACE_TRY(P->aval.alloc(es * nnz));
   if (P->prec == LACE_F64) {
     LACE_HIP(hipMemcpyAsync(P->aval.p, a64.p, sizeof(double) * nnz, hipMemcpyDeviceToDevice, stream()));
@@ -1136,15 +1141,15 @@ int ParILU::values_f64(double* lv, double* uv) {
   return DEV_SUCCESS;
 }
 
-int parilu_create(const data_d_matrix* A, lace_prec_t prec, ParILU** out) {
+int parilu_create(const data_d_matrix* A, lace_prec_t prec, ParILU** out, ParILUUse use) {
   LACE_TRY(ensure_init());
   LACE_REQUIRE(prec == LACE_F64 || prec == LACE_F32 || prec == LACE_BF16 || prec == LACE_F16,
                DEV_ERR_NOT_SUPPORTED, "ParILU precision %d not supported", (int)prec);
   auto* P = new ParILU();
   P->prec = prec;
-  int rc = build_pattern(A, P);
-  if (rc == DEV_SUCCESS) rc = P->reset();
-  if (rc == DEV_SUCCESS) rc = P->build_trsv();
+  int rc = build_pattern(A, P, use);
+  if (rc == DEV_SUCCESS && use.sweeps) rc = P->reset();
+  if (rc == DEV_SUCCESS && (use.jacobi || use.exact)) rc = P->build_trsv(use);
   if (rc != DEV_SUCCESS) {
     delete P;
     return rc;

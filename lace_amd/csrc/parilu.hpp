@@ -9,6 +9,14 @@
 
 namespace lace {
 
+// What a ParILU object is made for: sweeps, transposed solves, Jacobi and
+// exact solves.  A caller that knows which of these it will ask for (a solver
+// its kind of solve, a one-call entry point everything) has the others'
+// plans neither built nor uploaded.
+struct ParILUUse {
+  bool sweeps = true, trans = true, jacobi = true, exact = true;
+};
+
 // Marker of an unsolved row in the exact solves' solution vectors: a
 // signalling-NaN bit pattern, which arithmetic never produces (it yields
 // quiet NaNs).
@@ -101,11 +109,32 @@ struct TriPlan {
   DevBuf tperm, trow, tcol, tmap;
   mutable DevBuf tval, tsol;
   mutable const void* tval_src = nullptr;
+  // Exact solves in level order by one workgroup (trsv_ring.hip): the rows
+  // by level, each level's by falling length and padded to chunks of 64.
+  // rdesc holds a word pair per chunk, rperm the row at each slot (-1:
+  // padding), rslot each row's slot, ridx the off-diagonal operands' places
+  // in that order modulo 2^15, four to a group.  rspan is the farthest back
+  // an operand lies, which decides whether the solution's last rows fit in
+  // LDS.  rval / rdiag hold the values gathered from rval_src (cleared by
+  // refresh_strict), rrhs and rsol the right-hand side and the solution in
+  // that order.
+  int rchunks = 0;  // 0: no such form
+  int rgroups = 0;  // groups of four a row takes at most
+  int rspan = 0;
+  size_t rslots = 0;
+  DevBuf rdesc, rperm, rslot, ridx;
+  mutable DevBuf rval, rdiag, rrhs, rsol;
+  mutable const void* rval_src = nullptr;
   static constexpr unsigned kFormStrict = 1, kFormDiag = 2, kFormEll = 4, kFormDia = 8, kFormAll = 15;
   unsigned stale = 0;  // forms not yet gathered from strict_src
   size_t src_es = 0;   // element size of strict_src
-  int build(int n, const int* row, const int* col, bool upper);
-  int build_tiles(const int* row, const int* col);
+  // jacobi / exact: whether the forms of those solves are wanted; same: a
+  // plan of the same pattern and triangle, if there is one
+  int build(int n, const int* row, const int* col, bool upper, bool jacobi = true, bool exact = true,
+            const TriPlan* same = nullptr);
+  int build_tiles(const int* row, const int* col, bool exact);
+  int build_ring(const int* row, const int* col, const int* perm, const int* lptr);
+  int copy_ring(const TriPlan& o);
   int refresh_strict(const void* val, size_t elem_size);
   int ensure_forms(unsigned forms);
   // 16-bit diagonal form (fmt BF16 or F16) from the current FP32 forms,
@@ -116,6 +145,20 @@ struct TriPlan {
 // y = T^{-1} r, exact.  Level-scheduled: one launch per level.
 template <typename T>
 int tri_solve_levels(const TriPlan& P, const T* val, const T* r, T* y);
+// y = T^{-1} r, exact, by one workgroup in level order (trsv_ring.hip);
+// ring_ready: whether the plan holds that form, it fits T and it is expected
+// to beat the persistent kernel.
+template <typename T>
+bool ring_ready(const TriPlan& P);
+template <typename T>
+int tri_solve_ring(const TriPlan& P, const T* val, const T* r, T* y);
+// The same for two factors in a row, y = T2^{-1} T1^{-1} r: the vector
+// between them goes from one order to the other in one move (ring_pair:
+// whether both factors take that route).
+template <typename T>
+bool ring_pair(const TriPlan& P, const TriPlan& Q);
+template <typename T>
+int tri_solve_ring2(const TriPlan& P, const T* val, const TriPlan& Q, const T* val2, const T* r, T* y);
 // y = T^{-1} r, exact, one launch: rows run in level order and wait on the
 // rows they depend on (value slots are pre-filled with a NaN sentinel).
 template <typename T>
@@ -209,7 +252,7 @@ struct ParILU {
   double sweep_bytes() const;
   int get(data_d_matrix* L, data_d_matrix* U);
   int values_f64(double* lv, double* uv);
-  int build_trsv();
+  int build_trsv(ParILUUse use);
   int refresh_csr();
   // Everything a solve of this kind and direction reads (block: the
   // 32-column solves), current for the present factor values: L^T's values
@@ -222,6 +265,6 @@ struct ParILU {
   int apply(lace_trsv_kind_t kind, int sweeps, int trans, const void* r, void* z);
 };
 
-int parilu_create(const data_d_matrix* A, lace_prec_t prec, ParILU** out);
+int parilu_create(const data_d_matrix* A, lace_prec_t prec, ParILU** out, ParILUUse use = ParILUUse());
 
 }  // namespace lace

@@ -384,7 +384,9 @@ static int select_direction(Solver* S, int trans) {
   return DEV_SUCCESS;
 }
 
-static int solver_create(const data_d_matrix* A, const lace_solver_opts* o, Solver** out) {
+// given_factors: the caller loads L and U and solves forward only.
+static int solver_create(const data_d_matrix* A, const lace_solver_opts* o, Solver** out,
+                         bool given_factors = false) {
   LACE_TRY(ensure_init());
   LACE_REQUIRE(A && A->row && A->col && A->val && A->num_rows == A->num_cols, DEV_ERR_ILLEGAL_VALUE,
                "solver: A must be a square CSR or BCSR matrix");
@@ -434,7 +436,11 @@ static int solver_create(const data_d_matrix* A, const lace_solver_opts* o, Solv
     } else {
       LACE_REQUIRE(fp == LACE_F64 || fp == LACE_F32 || fp == LACE_BF16 || fp == LACE_F16, DEV_ERR_NOT_SUPPORTED,
                    "solver: CSR factor storage %d not supported", (int)fp);
-      LACE_TRY(parilu_create(A, fp, &S->P));
+      ParILUUse use;
+      use.sweeps = use.trans = !given_factors;
+      use.jacobi = o->trsv != LACE_TRSV_LEVEL;
+      use.exact = o->trsv != LACE_TRSV_JACOBI;
+      LACE_TRY(parilu_create(A, fp, &S->P, use));
       S->ilu = std::make_unique<PrecILU>(S->P, o->trsv, o->jacobi_sweeps, 0);
       base = S->ilu.get();
     }
@@ -1023,7 +1029,7 @@ int fgmres_dropin_common(data_d_matrix* A, data_d_matrix* b, data_d_matrix* x0, 
     o.restart_max = (int)((total + 62) / 63);
   }
   Solver* S = nullptr;
-  LACE_TRY(solver_create(A, &o, &S));
+  LACE_TRY(solver_create(A, &o, &S, true));
   std::unique_ptr<Solver> hold(S);
   if (get_option("matlab_log", 1) != 0) {
     MatlabLog& ml = S->mlog;

@@ -26,7 +26,8 @@
 namespace lace {
 
 // ---------------------------------------------------------------- plans
-int TriPlan::build(int n_, const int* row_, const int* col_, bool upper_) {
+int TriPlan::build(int n_, const int* row_, const int* col_, bool upper_, bool jacobi, bool exact,
+                   const TriPlan* same) {
   n = n_;
   nnz = row_[n_];
   upper = upper_;
@@ -45,6 +46,11 @@ int TriPlan::build(int n_, const int* row_, const int* col_, bool upper_) {
   LACE_TRY(upload(perm, perm_h.data(), sizeof(int) * std::max(n, 1)));
   LACE_TRY(upload(lptr, h_lptr.data(), sizeof(int) * (nlev + 1)));
   LACE_TRY(upload(sched, sched_h.data(), sizeof(int) * std::max(nslots, 1)));
+  strict_src = nullptr;
+  maxoff = 0;
+  for (int i = 0; i < n; i++) maxoff = std::max(maxoff, row_[i + 1] - row_[i] - 1);
+  if (exact) LACE_TRY(same ? copy_ring(*same) : build_ring(row_, col_, perm_h.data(), lptr_h.data()));
+  if (!jacobi) return build_tiles(row_, col_, exact);
   // off-diagonal form: every entry but the row's diagonal slot (first for
   // upper, last for lower), in row order
   std::vector<int> sr(n + 1, 0), sc, sm, dp(n);
@@ -68,7 +74,6 @@ int TriPlan::build(int n_, const int* row_, const int* col_, bool upper_) {
   // ELLPACK form for short rows
   int wmax = 0;
   for (int i = 0; i < n; i++) wmax = std::max(wmax, sr[i + 1] - sr[i]);
-  maxoff = wmax;
   ew = 0;
   if (n > 0 && wmax >= 1 && wmax <= 8 && (double)wmax * n <= 1.25 * snnz) {
     ew = wmax;
@@ -83,8 +88,7 @@ int TriPlan::build(int n_, const int* row_, const int* col_, bool upper_) {
   }
   // diagonal form of the same entries
   LACE_TRY(dia.build(n, row_, col_, [&](int i, int k) { return k != dp[i]; }));
-  strict_src = nullptr;
-  return build_tiles(row_, col_);
+  return build_tiles(row_, col_, exact);
 }
 
 // Grid dimensions under which every off-diagonal entry of the triangular
@@ -130,7 +134,7 @@ static bool tri_grid(int n, const int* row, const int* col, bool upper, long dim
   return true;
 }
 
-int TriPlan::build_tiles(const int* row_, const int* col_) {
+int TriPlan::build_tiles(const int* row_, const int* col_, bool exact) {
   tile_dims[0] = tile_dims[1] = tile_dims[2] = 0;
   grid[0] = grid[1] = grid[2] = 0;
   tval_src = nullptr;
@@ -139,6 +143,7 @@ int TriPlan::build_tiles(const int* row_, const int* col_) {
   const long full = (g[0] - 1) * g[1] * g[2] + g[0] * (g[1] - 1) * g[2] + g[0] * g[1] * (g[2] - 1);
   if (dia.nd == (g[2] > 1 ? 3 : 2) && snnz == full)
     for (int d = 0; d < 3; d++) grid[d] = (int)g[d];
+  if (!exact) return DEV_SUCCESS;
   // 512 rows per box: 8 x 8 x 8 in 3-D, 32 x 16 in 2-D (sides clipped to
   // the grid)
   const long want[3] = {g[2] > 1 ? 8 : 32, g[2] > 1 ? 8 : 16, 8};
@@ -207,6 +212,7 @@ int TriPlan::refresh_strict(const void* val, size_t es) {
   src_es = es;
   stale = kFormAll;
   tval_src = nullptr;
+  rval_src = nullptr;
   return DEV_SUCCESS;
 }
 
@@ -1408,14 +1414,16 @@ int tri_solve_persist_raw(int n, bool upper, const int* row, const int* col, con
                              nullptr, nullptr);
 }
 
-// Exact solve with a plan: the persistent kernel (option "trsv_exact" 1,
-// the default) with its blocks in box order where the plan has one (option
+// Exact solve with a plan: one workgroup in level order where that is
+// expected to be the fastest (ring_ready), else the persistent kernel
+// (option "trsv_exact" 1, the default) with its blocks in box order where the plan has one (option
 // "trsv_exact_tiles" 1), else blocks of consecutive rows, or the
 // level-ordered sync-free kernel (0).
 template <typename T>
 int tri_solve_exact(const TriPlan& P, const T* val, const T* r, T* y, unsigned* ticket, int* err) {
   if (get_option("trsv_exact", 1) == 0) return tri_solve_syncfree<T>(P, val, r, y, err);
   const double es = sizeof(T);
+  if (P.n > 0 && ring_ready<T>(P)) return tri_solve_ring<T>(P, val, r, y);
   const int wpc = get_option("trsv_exact_wgs_per_cu", 0), sleep = get_option("trsv_exact_poll_sleep", 0),
             rows = get_option("trsv_exact_rows", 512);
   const int slots = P.maxoff <= 4 ? 4 : kPersistR;
@@ -1687,10 +1695,10 @@ template int tri_solve_jacobi<float>(const TriPlan&, const float*, const float*,
                                       const float*, bool*, bool);
 
 // ---------------------------------------------------------------- ParILU solves
-int ParILU::build_trsv() {
-  LACE_TRY(lower.build(n, h_lrow.data(), h_lcol.data(), false));
+int ParILU::build_trsv(ParILUUse use) {
+  LACE_TRY(lower.build(n, h_lrow.data(), h_lcol.data(), false, use.jacobi, use.exact));
   lower.unit_diag = true;  // CSRL with the unit diagonal (never updated by sweeps)
-  LACE_TRY(lowerT.build(n, h_ucp.data(), h_uri.data(), false));
+  if (use.trans) LACE_TRY(lowerT.build(n, h_ucp.data(), h_uri.data(), false, use.jacobi, use.exact, sym ? &lower : nullptr));
   // U in CSR: transpose of the CSC arrays; map CSR slot -> CSC slot.
   {
     std::vector<int> r(n + 1, 0), c(nnzU), map(nnzU);
@@ -1703,11 +1711,11 @@ int ParILU::build_trsv() {
         c[q] = j;
         map[q] = p;
       }
-    LACE_TRY(upper.build(n, r.data(), c.data(), true));
+    LACE_TRY(upper.build(n, r.data(), c.data(), true, use.jacobi, use.exact));
     LACE_TRY(upload(u_csr_from_csc, map.data(), sizeof(int) * nnzU));
   }
   // L^T in CSR (diagonal first): transpose of L's CSR arrays.
-  {
+  if (use.trans) {
     std::vector<int> r(n + 1, 0), c(nnzL), map(nnzL);
     for (int p = 0; p < nnzL; p++) r[h_lcol[p] + 1]++;
     for (int i = 0; i < n; i++) r[i + 1] += r[i];
@@ -1718,13 +1726,13 @@ int ParILU::build_trsv() {
         c[q] = i;
         map[q] = p;
       }
-    LACE_TRY(upperT.build(n, r.data(), c.data(), true));
+    LACE_TRY(upperT.build(n, r.data(), c.data(), true, use.jacobi, use.exact, sym ? &upper : nullptr));
     upperT.unit_diag = true;
     LACE_TRY(upload(l_t_from_csr, map.data(), sizeof(int) * nnzL));
   }
   const size_t es = elem_size();
   LACE_TRY(uval_csr.alloc(es * nnzU));
-  LACE_TRY(lval_t.alloc(es * nnzL));
+  if (use.trans) LACE_TRY(lval_t.alloc(es * nnzL));
   LACE_TRY(work.alloc(es * n));
   LACE_TRY(work2.alloc(es * n));
   LACE_TRY(syncfree_err.alloc(sizeof(int) * 4));
@@ -1812,6 +1820,8 @@ static int apply_t(ParILU* P, lace_trsv_kind_t kind, int sweeps, int trans, cons
     return DEV_SUCCESS;
   }
   if (kind == LACE_TRSV_LEVEL) {
+    if (get_option("trsv_exact", 1) != 0 && P->n > 0 && ring_pair<T>(first, second))
+      return tri_solve_ring2<T>(first, v1, second, v2, r, z);
     int* err = P->syncfree_err.as<int>();
     unsigned* ticket = reinterpret_cast<unsigned*>(P->syncfree_err.as<int>() + 2);
     LACE_TRY(tri_solve_exact<T>(first, v1, r, tmp, ticket, err));
