@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "product_rows.hpp"
 
 using namespace lace;
 
@@ -827,31 +828,17 @@ int data_zfrobenius(data_d_matrix A, dataType* res) {
 // wraps mkl_sparse_spmm, blas/zspmm.cpp:47-167).  Dense-marker row merge.
 int data_z_spmm(dataType alpha, data_d_matrix A, data_d_matrix B, data_d_matrix* C) {
   const int m = A.num_rows, n = B.num_cols;
-  std::vector<int> mark(n, -1), list(n);
-  std::vector<double> acc(n, 0.0);
   std::vector<int> crow(m + 1, 0), ccol;
   std::vector<double> cval;
-  for (int i = 0; i < m; i++) {
-    int cnt = 0;
-    for (int p = A.row[i]; p < A.row[i + 1]; p++) {
-      int k = A.col[p];
-      for (int q = B.row[k]; q < B.row[k + 1]; q++) {
-        int j = B.col[q];
-        if (mark[j] != i) {
-          mark[j] = i;
-          list[cnt++] = j;
-          acc[j] = 0.0;
-        }
-        acc[j] += A.val[p] * B.val[q];
-      }
-    }
-    std::sort(list.begin(), list.begin() + cnt);
+  ccol.reserve((size_t)3 * (A.row[m] + (size_t)m));
+  cval.reserve((size_t)3 * (A.row[m] + (size_t)m));
+  product_rows(A, B, [&](int i, int cnt, const int* list, const double* acc) {
     for (int a = 0; a < cnt; a++) {
       ccol.push_back(list[a]);
       cval.push_back(alpha * acc[list[a]]);
     }
     crow[i + 1] = (int)ccol.size();
-  }
+  });
   free_arrays(C);
   C->storage_type = Magma_CSR;
   C->major = MagmaRowMajor;

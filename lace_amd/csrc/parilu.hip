@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "device.hpp"
 #include "parilu.hpp"
+#include "product_rows.hpp"
 
 namespace lace {
 
@@ -1291,15 +1292,13 @@ int data_zilures(data_d_matrix A, data_d_matrix L, data_d_matrix U, data_d_matri
   LACE_TRY(rc);
   double r = 0.0, nl = 0.0;
   for (int i = 0; i < n; i++) {
+    int lo = LU->row[i];
     for (int k = A.row[i]; k < A.row[i + 1]; k++) {
-      // LU rows are sorted: binary search for A's column
-      int lo = LU->row[i], hi = LU->row[i + 1];
-      int c = A.col[k];
-      while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (LU->col[mid] < c) lo = mid + 1;
-        else hi = mid;
-      }
+      // LU rows are sorted: on from the previous column's place, or from the
+      // row's start where A's columns are not in order
+      const int c = A.col[k];
+      if (k > A.row[i] && c < A.col[k - 1]) lo = LU->row[i];
+      while (lo < LU->row[i + 1] && LU->col[lo] < c) lo++;
       if (lo < LU->row[i + 1] && LU->col[lo] == c) {
         double t = LU->val[lo] - A.val[k];
         LU->val[lo] = t;
@@ -1318,6 +1317,36 @@ int data_zilures(data_d_matrix A, data_d_matrix L, data_d_matrix U, data_d_matri
 // ---------------------------------------------------------------- drop-ins
 namespace {
 
+// data_zilures's norms (L with its unit diagonal, U by columns) without
+// storing the product: a row at a time, the sums in the same order.
+int lu_residual(const data_d_matrix& A, const data_d_matrix& L, const data_d_matrix& U, double* res,
+                double* nonlinres) {
+  data_d_matrix Ur;
+  memset(&Ur, 0, sizeof(Ur));
+  LACE_TRY(data_zmconvert(U, &Ur, Magma_CSC, Magma_CSR));
+  double r = 0.0, nl = 0.0;
+  std::vector<double> row(Ur.num_cols);
+  product_rows(L, Ur, [&](int i, int cnt, const int* list, const double* acc) {
+    for (int a = 0; a < cnt; a++) row[a] = acc[list[a]];
+    int at = 0;
+    for (int k = A.row[i]; k < A.row[i + 1]; k++) {
+      const int c = A.col[k];
+      if (k > A.row[i] && c < A.col[k - 1]) at = 0;
+      while (at < cnt && list[at] < c) at++;
+      if (at < cnt && list[at] == c) {
+        const double t = row[at] - A.val[k];
+        row[at] = t;
+        nl += t * t;
+      }
+    }
+    for (int a = 0; a < cnt; a++) r += row[a] * row[a];
+  });
+  data_zmfree(&Ur);
+  *res = std::sqrt(r);
+  *nonlinres = std::sqrt(nl);
+  return DEV_SUCCESS;
+}
+
 // Shared body of the ParILU drop-ins.  mode 0: stop when step <=
 // reduction*Ares or after 20 sweeps (src/parilu_v0_3.cpp:44-45,62);
 // mode 1: stop after log->maxSweeps sweeps or when step <= 4 eps
@@ -1332,16 +1361,13 @@ int parilu_dropin(data_d_matrix* A, data_d_matrix* L, data_d_matrix* U, double r
   U->diagorder_type = Magma_VALUE;
   LACE_TRY(data_zmconvert(*A, U, Magma_CSR, Magma_CSCU));
   double Ares = 0.0, Anl = 0.0;
-  data_d_matrix LU;
-  memset(&LU, 0, sizeof(LU));
-  LACE_TRY(data_zilures(*A, *L, *U, &LU, &Ares, &Anl));
-  data_zmfree(&LU);
+  LACE_TRY(lu_residual(*A, *L, *U, &Ares, &Anl));
   double anorm = 0.0;
   LACE_TRY(data_zfrobenius(*A, &anorm));
   LACE_TRY(data_rowindex(A, &A->rowidx));
   ParILU* P = nullptr;
   auto t0 = std::chrono::steady_clock::now();
-  LACE_TRY(parilu_create(A, LACE_F64, &P));
+  LACE_TRY(parilu_create(A, LACE_F64, &P, ParILUUse{true, false, false, false}));
   const double tol = reduction * Ares;
   int iter = 0;
   double step = 3.402823466e+38;  // FLT_MAX, as the reference starts
