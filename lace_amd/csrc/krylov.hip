@@ -24,6 +24,7 @@
 // the device in one-workgroup kernels; the host only reads the convergence
 // flag.  Every kernel after the first of a cycle returns at once when the
 // device-side done flag is set, so a caller may queue steps ahead.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -115,59 +116,106 @@ __global__ __launch_bounds__(kBS) void mdot_kernel(int n, int ld, const K* __res
   }
 }
 
-// The same multi-dot with the slab's rows split over the block's threads.
-// A whole slab of R * 256 rows (every block but those cut by rowstart or
-// the end when R > 0) keeps its w rows in registers, R per thread as 16-byte
-// words of V consecutive rows (thread t: words t, t + 256, ...), and walks
-// the columns one after another: each column's slab is one contiguous run
-// read as 16-byte words, one column at a time per wave, and w is read once
-// for all columns.  Measured on FP64 n = 2^21, 50 columns: 6.1 TB/s against
-// 3.4 TB/s for rows outer and 16 columns inner with single-row loads.  Other
-// slabs take the rows-outer form: thread t takes the groups of V rows t,
-// t + 256, ... and loads each column's V rows and w's as one 16-byte word
-// (single rows for FP64 chunks of 16 columns, whose two-row form would hold
-// 32 doubles of U per thread), the columns in chunks of NC in registers
-// with w's slab read again per chunk, from cache.  U, w and ld must be
-// 16-byte aligned (the engine's buffers are); groups cut by rowstart or the
-// slab end load element by element.
+// The same multi-dot with the slab's rows split over the block's threads
+// and, where slabs alone leave CUs idle, the columns over blockIdx.y (cpb
+// columns each).  Slabs of R * 256 rows (R > 0) keep their w rows in
+// registers, R per thread as 16-byte words of consecutive rows (thread t:
+// words t, t + 256, ...), and walk the columns in groups whose loads are all
+// issued before any is used: each column's slab is one contiguous run, and w
+// is read once for all columns.  Rows outside [rowstart, n) count as zeros of
+// w; columns are padded with zeros up to ld, a multiple of 64.  Slabs of
+// another length (R = 0) take the rows-outer form: thread t takes the groups
+// of V rows t, t + 256, ... and loads each column's V rows and w's as one
+// 16-byte word (single rows for FP64 chunks of 16 columns, whose two-row form
+// would hold 32 doubles of U per thread), the columns in chunks of NC in
+// registers with w's slab read again per chunk, from cache; groups cut by
+// rowstart or the slab end load element by element.  U, w and ld must be
+// 16-byte aligned (the engine's buffers are).  FP64, 50 columns: 2^21 rows
+// 6.1 TB/s (rows outer with single-row loads: 3.4); 262144 rows, 23
+// columns on average, 17.7 -> 11.4 us, and with a first slab cut by rowstart,
+// which took the rows-outer form and held up the launch, 29.7 -> 12.5 us (41
+// columns).
 template <typename K, int NC, bool SELF, int R>
 __global__ __launch_bounds__(kBS, 4) void mdot_rows_kernel(int n, int ld, const K* __restrict__ U, int ncols,
                                                         const K* __restrict__ w, int rowstart, int rpb,
-                                                        double* __restrict__ partial, int pstride,
+                                                        int cpb, double* __restrict__ partial, int pstride,
                                                         const double* __restrict__ misc) {
   if (misc && is_done(misc)) return;
   constexpr int V = (sizeof(K) == 8 && NC > 8) ? 1 : 16 / (int)sizeof(K);
   constexpr int VW = 16 / (int)sizeof(K);  // rows per 16-byte word
   constexpr int RW = R > 0 ? R / VW : 1;   // w words per thread on the register path
+  constexpr int CG = RW >= 4 ? 2 : NC;     // columns whose loads are in flight together
   const int b = xcd_block(blockIdx.x, gridDim.x);
   const int r0 = max(b * rpb, rowstart), r1 = min((b + 1) * rpb, n);
+  const int cend = min(ncols, ((int)blockIdx.y + 1) * cpb);
   const int wave = threadIdx.x >> 6;
-  const bool whole = R > 0 && rpb == R * kBS && r0 == b * rpb && r1 == (b + 1) * rpb;
   K wr[RW][VW];
-  if (whole) {
+  unsigned row[RW];
+  bool in[RW];
+  if constexpr (R > 0) {
 #pragma unroll
-    for (int i = 0; i < RW; i++) vload<K, VW>(w + r0 + (size_t)(threadIdx.x + kBS * i) * VW, wr[i]);
+    for (int i = 0; i < RW; i++) {
+      const int i0 = b * rpb + ((int)threadIdx.x + kBS * i) * VW;
+      row[i] = (unsigned)i0;
+      in[i] = i0 < n;
+      if (i0 >= r0 && i0 + VW <= r1) {
+        vload<K, VW>(w + i0, wr[i]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VW; e++) wr[i][e] = (i0 + e >= r0 && i0 + e < r1) ? w[i0 + e] : K(0);
+      }
+    }
   }
   __shared__ double red[kBS / 64][NC + 1];
   // at least one pass, for the SELF sum when there are no columns
-  for (int c0 = 0; c0 < ncols || (c0 == 0 && SELF); c0 += NC) {
-    const int nck = min(NC, ncols - c0);
+  for (int c0 = blockIdx.y * cpb; c0 < cend || (c0 == 0 && SELF); c0 += NC) {
+    const int nck = min(NC, cend - c0);
     const bool self_pass = SELF && c0 == 0;
     K acc[NC];
     K self = K(0);
 #pragma unroll
     for (int k = 0; k < NC; k++) acc[k] = K(0);
-    if (whole) {
+    if constexpr (R > 0) {
 #pragma unroll
-      for (int k = 0; k < NC; k++) {
-        if (k < nck) {
-          const K* col = U + (size_t)(c0 + k) * ld + r0;
+      for (int g = 0; g < NC; g += CG) {
+        if (g + CG <= nck) {
+          K uv[CG][RW][VW];
 #pragma unroll
-          for (int i = 0; i < RW; i++) {
-            K uv[VW];
-            vload<K, VW>(col + (size_t)(threadIdx.x + kBS * i) * VW, uv);
+          for (int k = 0; k < CG; k++)
 #pragma unroll
-            for (int e = 0; e < VW; e++) acc[k] += uv[e] * wr[i][e];
+            for (int i = 0; i < RW; i++) {
+              if (in[i]) {
+                vload<K, VW>(U + (size_t)(c0 + g + k) * ld + row[i], uv[k][i]);
+              } else {
+#pragma unroll
+                for (int e = 0; e < VW; e++) uv[k][i][e] = K(0);
+              }
+            }
+#pragma unroll
+          for (int k = 0; k < CG; k++)
+#pragma unroll
+            for (int i = 0; i < RW; i++)
+#pragma unroll
+              for (int e = 0; e < VW; e++) acc[g + k] += uv[k][i][e] * wr[i][e];
+        } else {
+#pragma unroll
+          for (int k = g; k < g + CG; k++) {
+            if (k < nck) {
+              K uv[RW][VW];
+#pragma unroll
+              for (int i = 0; i < RW; i++) {
+                if (in[i]) {
+                  vload<K, VW>(U + (size_t)(c0 + k) * ld + row[i], uv[i]);
+                } else {
+#pragma unroll
+                  for (int e = 0; e < VW; e++) uv[i][e] = K(0);
+                }
+              }
+#pragma unroll
+              for (int i = 0; i < RW; i++)
+#pragma unroll
+                for (int e = 0; e < VW; e++) acc[k] += uv[i][e] * wr[i][e];
+            }
           }
         }
       }
@@ -226,9 +274,10 @@ __global__ __launch_bounds__(kBS, 4) void mdot_rows_kernel(int n, int ld, const 
   }
 }
 
-// Launches the multi-dot: the register path for whole slabs of 1024 or
-// 2048 rows (8 columns per pass), the rows-outer form otherwise (NC columns
-// per pass).
+// Launches the multi-dot: the register path for slabs of 1024 or 2048 rows
+// (8 columns per pass), the rows-outer form otherwise (NC columns per pass).
+// The register path's columns go over blockIdx.y in multiples of 8 until
+// there are 2048 blocks (8 per CU).
 // The step's first multi-dot (U_j^T w, no self term) is the timing region
 // "hh_mdot" with its algorithmic bytes, every column and w once.
 template <typename K, int NC, bool SELF>
@@ -236,15 +285,18 @@ static void launch_mdot_rows(const HHEngine<K>& E, const K* U, int ncols, const 
                              double* part, const double* misc) {
   TimedRegion tr(SELF ? "hh_mdot_self" : "hh_mdot", 0.0,
                  (double)sizeof(K) * (double)(E.n - rowstart) * (double)(ncols + 1), true);
+  const int chunks = std::max(1, ceil_div(ncols, 8));
+  const int cpb = ceil_div(chunks, std::max(1, std::min(chunks, 2048 / E.nb))) * 8;
+  const dim3 grid(E.nb, std::max(1, ceil_div(ncols, cpb)));
   if (E.rpb == 8 * kBS)
-    tr.launch(mdot_rows_kernel<K, 8, SELF, 8>, dim3(E.nb), dim3(kBS), E.n, E.ld, U, ncols, w, rowstart, E.rpb,
+    tr.launch(mdot_rows_kernel<K, 8, SELF, 8>, grid, dim3(kBS), E.n, E.ld, U, ncols, w, rowstart, E.rpb, cpb,
               part, E.pstride, misc);
   else if (E.rpb == 4 * kBS)
-    tr.launch(mdot_rows_kernel<K, 8, SELF, 4>, dim3(E.nb), dim3(kBS), E.n, E.ld, U, ncols, w, rowstart, E.rpb,
+    tr.launch(mdot_rows_kernel<K, 8, SELF, 4>, grid, dim3(kBS), E.n, E.ld, U, ncols, w, rowstart, E.rpb, cpb,
               part, E.pstride, misc);
   else
     tr.launch(mdot_rows_kernel<K, NC, SELF, 0>, dim3(E.nb), dim3(kBS), E.n, E.ld, U, ncols, w, rowstart, E.rpb,
-              part, E.pstride, misc);
+              ncols, part, E.pstride, misc);
 }
 
 // Column totals of the per-block partials when there are many columns: one
@@ -268,22 +320,25 @@ __global__ __launch_bounds__(256) void reduce_cols_kernel(int nb, int cnt, int s
 }
 
 // Sum of the per-block partials in a fixed order: out[k] for k < cnt and,
-// if self, out[cnt] = the self slot.  One block of 256 threads, ch columns
+// if self, out[cnt] = the self slot.  One block of BS threads, ch columns
 // at a time (ch: the column count rounded up to a power of two, at most
-// 16): lane t reads column t % ch of the partial rows t / ch, t / ch +
-// 256 / ch, ..., so the lanes of a row read its consecutive words and a
+// 64): lane t reads column t % ch of the partial rows t / ch, t / ch +
+// BS / ch, ..., so the lanes of a row read its consecutive words and a
 // round touches each cache line once, and a thread issues the loads of 64
-// of its rows before adding any of them, so the 1024 rows of a 2M-row
-// vector's 2048-row slabs take one wait for memory.  The row groups' sums
-// then meet in a fixed butterfly per wave and a fixed 4-wave combination.
+// (BS 1024: 16) of its rows before adding any of them, so the 1024 rows of a
+// 2M-row vector's 2048-row slabs take one wait for memory.  The row groups' sums
+// then meet in a fixed butterfly per wave and a fixed combination of the
+// waves.
+template <int BS>
 __device__ __forceinline__ void finalize_partials(int nb, int cnt, bool self, int pstride,
                                                   const double* __restrict__ partial, double* out) {
-  constexpr int RB = 64;  // rows in flight per thread
-  __shared__ double seg[kBS / 64][16];
+  constexpr int RB = BS >= 1024 ? 16 : 64;  // rows in flight per thread
+  constexpr int CH = BS >= 1024 ? 64 : 16;
+  __shared__ double seg[BS / 64][CH];
   const int tot = cnt + (self ? 1 : 0);
   int ch = 1;
-  while (ch < tot && ch < 16) ch <<= 1;
-  const int G = kBS / ch;  // row groups
+  while (ch < tot && ch < CH) ch <<= 1;
+  const int G = BS / ch;  // row groups
   const int k = threadIdx.x & (ch - 1), g = threadIdx.x / ch;
   const int wv = threadIdx.x >> 6;
   for (int base = 0; base < tot; base += ch) {
@@ -306,9 +361,12 @@ __device__ __forceinline__ void finalize_partials(int nb, int cnt, bool self, in
     for (int off = ch; off < 64; off <<= 1) acc += __shfl_xor(acc, off);
     if ((int)(threadIdx.x & 63) < ch) seg[wv][k] = acc;
     __syncthreads();
-    if ((int)threadIdx.x < ch && base + (int)threadIdx.x < tot)
-      out[base + threadIdx.x] = (seg[0][threadIdx.x] + seg[1][threadIdx.x]) +
-                                (seg[2][threadIdx.x] + seg[3][threadIdx.x]);
+    if ((int)threadIdx.x < ch && base + (int)threadIdx.x < tot) {
+      double t[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < BS / 64; q++) t[q & 3] += seg[q][threadIdx.x];
+      out[base + threadIdx.x] = (t[0] + t[1]) + (t[2] + t[3]);
+    }
     __syncthreads();
   }
 }
@@ -322,7 +380,7 @@ __global__ __launch_bounds__(256) void hh_start_kernel(int nb, int pstride, cons
                                                        SmallLayout lay, int set_rtol, double rtol_rel) {
   double* misc = small + lay.misc();
   __shared__ double nu[1];
-  finalize_partials(nb, 0, true, pstride, partial, nu);
+  finalize_partials<256>(nb, 0, true, pstride, partial, nu);
   __syncthreads();
   if (threadIdx.x == 0) {
     const double rnorm = sqrt(nu[0]);
@@ -364,48 +422,96 @@ __global__ __launch_bounds__(kBS) void hh_start_vec_kernel(int n, const K* __res
 // ------------------------------------------------------------ step kernels
 // The one-workgroup kernels below stage the small dense state they loop
 // over (T, the Hessenberg column, the rotations) in LDS with parallel
-// loads first, so their O(j) loops never wait on a global load.
+// loads first, so their O(j) loops never wait on a global load: all loads,
+// the done flag's among them, are issued together, before the sum of the
+// partials whose wait then covers them (a finished cycle's partials are
+// stale but in bounds, and nothing is written before the flag is tested).
+constexpr int kSmallBS = 1024;
 constexpr int kMaxT = 65 * 65;  // T for restart lengths up to 63
+constexpr int kTRegs = (kMaxT + kSmallBS - 1) / kSmallBS;
 
-__device__ __forceinline__ void stage(const double* __restrict__ src, int count, double* dst) {
-  for (int e = threadIdx.x; e < count; e += blockDim.x) dst[e] = src[e];
-}
+// T's first nc columns: into registers, and from there into LDS with an odd
+// leading dimension (a row of lanes then falls on different banks).
+struct TStage {
+  double v[kTRegs];
+  __device__ __forceinline__ void load(const double* __restrict__ T, int ldT, int nc) {
+#pragma unroll
+    for (int q = 0; q < kTRegs; q++) {
+      const int e = threadIdx.x + kSmallBS * q;
+      v[q] = e < nc * ldT ? T[e] : 0.0;
+    }
+  }
+  __device__ __forceinline__ void store(double* Ts, int ldT, int nc) const {
+#pragma unroll
+    for (int q = 0; q < kTRegs; q++) {
+      const int e = threadIdx.x + kSmallBS * q;
+      if (e < nc * ldT) Ts[e % ldT + (e / ldT) * (ldT | 1)] = v[q];
+    }
+  }
+};
 
 // c = U_j^T w (from partials); d = T_j^T c.
-__global__ __launch_bounds__(256) void hh_dT_kernel(int nb, int pstride, const double* partial, int j,
-                                                    double* small, SmallLayout lay) {
-  double* misc = small + lay.misc();
-  if (is_done(misc)) return;
+__global__ __launch_bounds__(kSmallBS) void hh_dT_kernel(int nb, int pstride, const double* partial, int j,
+                                                         double* small, SmallLayout lay) {
+  const bool done = is_done(small + lay.misc());
   __shared__ double c[72];
-  __shared__ double Ts[kMaxT];
-  const int ldT = lay.ldT();
-  stage(small + lay.T(), (j + 1) * ldT, Ts);
-  finalize_partials(nb, j + 1, false, pstride, partial, c);
+  __shared__ double Ts[kMaxT + 65];
+  const int ldT = lay.ldT(), lds = ldT | 1;
+  TStage st;
+  st.load(small + lay.T(), ldT, j + 1);
+  finalize_partials<kSmallBS>(nb, j + 1, false, pstride, partial, c);
+  st.store(Ts, ldT, j + 1);
   __syncthreads();
-  double* d = small + lay.d();
-  for (int k = threadIdx.x; k <= j; k += 256) {
+  if (done) return;
+  const int k = threadIdx.x;
+  if (k <= j) {
     double v = 0.0;
-    for (int l = 0; l <= k; l++) v += Ts[l + k * ldT] * c[l];
-    d[k] = v;
+#pragma unroll 8
+    for (int l = 0; l <= k; l++) v += Ts[l + k * lds] * c[l];
+    small[lay.d() + k] = v;
   }
 }
 
-// w <- w - U_j d.
-template <typename K, int NC>
+// v <- v - U d on the V rows at i0, columns in ascending order; the loads
+// of eight columns are issued before the first is used (one column at a time
+// leaves a small matrix waiting on each: 64 x 64 points, 17 to 50
+// columns, 6.4 -> 4.2 us; 262144 rows 13.0 -> 11.6 us).
+template <typename K, int V, int B>
+__device__ __forceinline__ void sub_cols(const K* __restrict__ U, int ld, int i0, int k0,
+                                         const double* __restrict__ d, K (&v)[V]) {
+  K u[B][V];
+#pragma unroll
+  for (int q = 0; q < B; q++) wload<K, V>(U + (size_t)(k0 + q) * ld + i0, u[q]);
+#pragma unroll
+  for (int q = 0; q < B; q++)
+#pragma unroll
+    for (int e = 0; e < V; e++) v[e] -= u[q][e] * (K)d[k0 + q];
+}
+template <typename K, int V>
+__device__ __forceinline__ void sub_all(const K* __restrict__ U, int ld, int i0, int ncols,
+                                        const double* __restrict__ d, K (&v)[V]) {
+  int k = 0;
+  for (; k + 8 <= ncols; k += 8) sub_cols<K, V, 8>(U, ld, i0, k, d, v);
+  if (ncols & 4) sub_cols<K, V, 4>(U, ld, i0, k, d, v), k += 4;
+  if (ncols & 2) sub_cols<K, V, 2>(U, ld, i0, k, d, v), k += 2;
+  if (ncols & 1) sub_cols<K, V, 1>(U, ld, i0, k, d, v);
+}
+
+// w <- w - U_j d, a 16-byte word of rows per thread (the rows past n of the
+// last one are padding: ld is a multiple of 64).
+template <typename K>
 __global__ __launch_bounds__(kBS) void hh_update_kernel(int n, int ld, const K* __restrict__ U, int ncols,
                                                         const double* __restrict__ small, SmallLayout lay,
                                                         K* __restrict__ w) {
+  constexpr int V = 16 / (int)sizeof(K);
   const double* misc = small + lay.misc();
-  if (is_done(misc)) return;
   const int b = xcd_block(blockIdx.x, gridDim.x);
-  const int i = b * kBS + threadIdx.x;
-  if (i >= n) return;
-  const double* d = small + lay.d();
-  K v = w[i];
-#pragma unroll
-  for (int k = 0; k < NC; k++)
-    if (k < ncols) v -= U[(size_t)k * ld + i] * (K)d[k];
-  w[i] = v;
+  const int i0 = (b * kBS + (int)threadIdx.x) * V;
+  if (i0 >= n || is_done(misc)) return;
+  K v[V];
+  wload<K, V>(w + i0, v);
+  sub_all<K, V>(U, ld, i0, ncols, small + lay.d(), v);
+  wstore<K, V>(w + i0, v);
 }
 
 // w <- w - U_j d and, from the updated rows >= rowstart, the tail
@@ -495,42 +601,62 @@ __global__ __launch_bounds__(kBS) void hh_update_mdot_kernel(int n, int ld, cons
 // Hessenberg column j rotated by the previous Givens rotations; new
 // rotation (src/givens.cpp:46-67 with tol = the smallest subnormal);
 // residual estimate |g_{j+1}|; y' = T_{j+1} U_{j+1}^T e_{j+1} for q.
+// The rotations' serial chain runs on the second wave, beside the products
+// with T on the first.
 template <typename K>
-__global__ __launch_bounds__(256) void hh_newcol_small_kernel(int nb, int pstride, const double* partial,
-                                                              int j, int n, int ld,
-                                                              const K* __restrict__ U,
-                                                              const K* __restrict__ w, double* small,
-                                                              SmallLayout lay) {
+__global__ __launch_bounds__(kSmallBS) void hh_newcol_small_kernel(int nb, int pstride, const double* partial,
+                                                                   int j, int n, int ld,
+                                                                   const K* __restrict__ U,
+                                                                   const K* __restrict__ w, double* small,
+                                                                   SmallLayout lay) {
   double* misc = small + lay.misc();
-  if (is_done(misc)) return;
+  const bool done = is_done(misc);
   __shared__ double s[72];
   __shared__ double e[72];
+  __shared__ double u[72];   // U_j^T u_{j+1}
   __shared__ double h[72];   // Hessenberg column j
   __shared__ double cz[72];  // previous rotations
   __shared__ double sz[72];
-  __shared__ double sc[4];
-  __shared__ double Ts[kMaxT];
+  __shared__ double sc[6];
+  __shared__ double Ts[kMaxT + 65];
   double* T = small + lay.T();
-  const int ldT = lay.ldT();
+  const int ldT = lay.ldT(), lds = ldT | 1;
   const int j1 = j + 1;
-  const double* cs = small + lay.cs();
-  const double* sn = small + lay.sn();
-  // parallel staging: T's first j+1 columns, w'[0..j], the rotations, and
-  // row j+1 of the reflectors
-  stage(T, j1 * ldT, Ts);
-  for (int i = threadIdx.x; i <= j; i += 256) {
-    h[i] = (double)w[i];
-    e[i] = j1 < n ? (double)U[(size_t)i * ld + j1] : 0.0;
-    if (i < j) {
-      cz[i] = cs[i];
-      sz[i] = sn[i];
+  const int t = threadIdx.x;
+  // staging: T's first j+1 columns, w'[0..j], the rotations, row j+1 of the
+  // reflectors, w'[j+1], g_j and the tolerance
+  TStage st;
+  st.load(T, ldT, j1);
+  double hv = 0.0, ev = 0.0, cv = 0.0, sv = 0.0, x = 0.0;
+  if (t <= j) {
+    hv = (double)w[t];
+    ev = j1 < n ? (double)U[(size_t)t * ld + j1] : 0.0;
+    if (t < j) {
+      cv = small[lay.cs() + t];
+      sv = small[lay.sn() + t];
     }
+  } else if (t == 64) {
+    x = j1 < n ? (double)w[j1] : 0.0;
+  } else if (t == 65) {
+    x = small[lay.g() + j];
+  } else if (t == 66) {
+    x = misc[MS_RTOL];
   }
-  finalize_partials(nb, j + 1, true, pstride, partial, s);  // s[0..j], s[j+1] = nu
+  finalize_partials<kSmallBS>(nb, j + 1, true, pstride, partial, s);  // s[0..j], s[j+1] = nu
+  st.store(Ts, ldT, j1);
+  if (t <= j) {
+    h[t] = hv;
+    e[t] = ev;
+    cz[t] = cv;
+    sz[t] = sv;
+  } else if (t >= 64 && t < 67) {
+    sc[3 + t - 64] = x;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (done) return;
+  if (t == 0) {
     const double nu = s[j1];
-    const double alpha = j1 < n ? (double)w[j1] : 0.0;
+    const double alpha = sc[3];
     const double sq = sqrt(nu);
     const double dd = (alpha >= 0.0 ? 1.0 : -1.0) * sq;
     const double nv = sqrt(2.0 * sq * (sq + fabs(alpha)));
@@ -545,96 +671,108 @@ __global__ __launch_bounds__(256) void hh_newcol_small_kernel(int nb, int pstrid
   }
   __syncthreads();
   const double dd = sc[0], scale = sc[1];
-  // utu = U_j^T u_{j+1} = scale * (s + dd * e[0..j]); T[0..j, j+1] = -2 T_j utu
-  for (int l = threadIdx.x; l <= j1; l += 256) {
-    double v = 2.0;
-    if (l <= j) {
-      v = 0.0;
-      for (int k = l; k <= j; k++) v += Ts[l + k * ldT] * (scale * (s[k] + dd * e[k]));
-      v = -2.0 * v;
-    }
-    Ts[l + j1 * ldT] = v;
-    T[l + j1 * ldT] = v;
-  }
+  // U_j^T u_{j+1} = scale * (s + dd * e[0..j])
+  if (t <= j) u[t] = scale * (s[t] + dd * e[t]);
   __syncthreads();
-  // y' = T_{j+1} e
-  double* yq = small + lay.y();
-  for (int l = threadIdx.x; l <= j1; l += 256) {
-    double v = 0.0;
-    for (int k = l; k <= j1; k++) v += Ts[l + k * ldT] * e[k];
-    yq[l] = v;
-  }
-  if (threadIdx.x == 0) {
-    double* csw = small + lay.cs();
-    double* snw = small + lay.sn();
+  if (t < 64) {
+    // T[0..j, j+1] = -2 T_j u, then y' = T_{j+1} e
+    if (t <= j1) {
+      double v = 2.0, y = 0.0;
+      if (t <= j) {
+        v = 0.0;
+#pragma unroll 8
+        for (int k = t; k <= j; k++) {
+          const double tk = Ts[t + k * lds];
+          v += tk * u[k];
+          y += tk * e[k];
+        }
+        v = -2.0 * v;
+      }
+      T[t + j1 * ldT] = v;
+      small[lay.y() + t] = y + v * e[j1];
+    }
+  } else if (t == 64) {
     double* g = small + lay.g();
     // Hessenberg column: h_i = w'_i (i <= j), h_{j+1} = -dd; apply the
     // previous rotations
+    double t0 = h[0];
+#pragma unroll 8
     for (int i = 0; i < j; i++) {
-      const double t0 = h[i], t1 = h[i + 1];
-      h[i + 1] = -sz[i] * t0 + cz[i] * t1;
+      const double t1 = h[i + 1];
+      const double n1 = -sz[i] * t0 + cz[i] * t1;
       h[i] = cz[i] * t0 + sz[i] * t1;
+      t0 = n1;
     }
-    const double a = h[j], bb = -dd;
+    const double a = t0, bb = -dd;
     const double tol = 4.9406564584124654e-324;  // nextafter(0,1)
     double c, sn_;
     if (fabs(bb) <= tol) {
       c = 1.0;
       sn_ = 0.0;
     } else if (fabs(bb) > fabs(a)) {
-      const double t = a / bb;
-      sn_ = 1.0 / sqrt(1.0 + t * t);
-      c = t * sn_;
+      const double q = a / bb;
+      sn_ = 1.0 / sqrt(1.0 + q * q);
+      c = q * sn_;
     } else {
-      const double t = bb / a;
-      c = 1.0 / sqrt(1.0 + t * t);
-      sn_ = t * c;
+      const double q = bb / a;
+      c = 1.0 / sqrt(1.0 + q * q);
+      sn_ = q * c;
     }
-    csw[j] = c;
-    snw[j] = sn_;
+    small[lay.cs() + j] = c;
+    small[lay.sn() + j] = sn_;
     h[j] = c * a - sn_ * dd;
-    const double gj = g[j];
-    g[j1] = -sn_ * gj;
+    const double gj = sc[4];
+    const double gn = -sn_ * gj;
+    g[j1] = gn;
     g[j] = c * gj;
-    const double res = fabs(g[j1]);
+    const double res = fabs(gn);
     misc[MS_RES] = res;
     misc[MS_NCOLS] = (double)j1;
-    if (!(res >= misc[MS_RTOL]) || !isfinite(res)) misc[MS_DONE] = 1.0;
+    if (!(res >= sc[5]) || !isfinite(res)) misc[MS_DONE] = 1.0;
     if (!isfinite(res)) misc[MS_BREAK] = 1.0;
   }
   __syncthreads();
   // rotated Hessenberg column -> R
-  double* R = small + lay.R();
-  const int ldR = lay.m + 1;
-  for (int i = threadIdx.x; i <= j; i += 256) R[i + j * ldR] = h[i];
+  if (t <= j) small[lay.R() + t + j * (lay.m + 1)] = h[t];
 }
 
 // u_{j+1} = (w + dd e_{j+1}) * scale on rows >= j+1 (0 above);
-// q = e_{j+1} - U_{j+1} y'.
-template <typename K, int NC>
+// q = e_{j+1} - U_{j+1} y'.  A 16-byte word of rows per thread; rows past n
+// are written as zeros of u (and not read from w).
+template <typename K>
 __global__ __launch_bounds__(kBS) void hh_newcol_vec_kernel(int n, int ld, K* __restrict__ U, int j,
                                                             const K* __restrict__ w,
                                                             const double* __restrict__ small,
                                                             SmallLayout lay, K* __restrict__ q,
                                                             int write_q) {
+  constexpr int V = 16 / (int)sizeof(K);
   const double* misc = small + lay.misc();
-  if (is_done(misc)) return;
   const int b = xcd_block(blockIdx.x, gridDim.x);
-  const int i = b * kBS + threadIdx.x;
-  if (i >= n) return;
+  const int i0 = (b * kBS + (int)threadIdx.x) * V;
+  if (i0 >= n || is_done(misc)) return;
   const int j1 = j + 1;
+  K wv[V];
+  if (i0 + V <= n) {
+    wload<K, V>(w + i0, wv);
+  } else {
+#pragma unroll
+    for (int e = 0; e < V; e++) wv[e] = i0 + e < n ? w[i0 + e] : K(0);
+  }
   const double dd = misc[MS_DD], scale = misc[MS_SCALE];
-  K unew = K(0);
-  if (i >= j1) unew = (K)(((double)w[i] + (i == j1 ? dd : 0.0)) * scale);
-  U[(size_t)j1 * ld + i] = unew;
+  K unew[V], v[V];
+#pragma unroll
+  for (int e = 0; e < V; e++) {
+    const int i = i0 + e;
+    unew[e] = i >= j1 && i < n ? (K)(((double)wv[e] + (i == j1 ? dd : 0.0)) * scale) : K(0);
+    v[e] = i == j1 ? K(1) : K(0);
+  }
+  wstore<K, V>(U + (size_t)j1 * ld + i0, unew);
   if (!write_q) return;
   const double* yq = small + lay.y();
-  K v = (i == j1) ? K(1) : K(0);
+  sub_all<K, V>(U, ld, i0, j1, yq, v);
 #pragma unroll
-  for (int k = 0; k < NC; k++)
-    if (k <= j) v -= U[(size_t)k * ld + i] * (K)yq[k];
-  v -= unew * (K)yq[j1];
-  q[i] = v;
+  for (int e = 0; e < V; e++) v[e] -= unew[e] * (K)yq[j1];
+  wstore<K, V>(q + i0, v);
 }
 
 // Least squares y = R^{-1} g by the column-oriented back substitution of
@@ -804,9 +942,10 @@ int hh_start(HHEngine<K>& E, int set_rtol, double rtol_rel) {
   return DEV_SUCCESS;
 }
 
-// Householder part of step j (after w = A z_j).  Beyond 16 columns the
-// per-block partials are first reduced column by column on many
-// workgroups, and the one-workgroup kernels read the totals.
+// Householder part of step j (after w = A z_j).  Beyond 16 columns of more
+// than 512 slabs the per-block partials are first reduced column by column
+// on many workgroups, and the one-workgroup kernels read the totals (fewer
+// are summed by the one workgroup in the time that launch would take).
 template <typename K>
 int hh_step(HHEngine<K>& E, int j, bool write_q) {
   TimedRegion tr("householder");
@@ -817,14 +956,14 @@ int hh_step(HHEngine<K>& E, int j, bool write_q) {
   double* part = E.partial.template as<double>();
   double* ptot = E.ptot.template as<double>();
   const double* misc = small + E.lay.misc();
-  const int nbv = ceil_div(E.n, kBS);
-  const bool wide = nc > 16;
+  const int nbv = ceil_div(E.n, kBS * 16 / (int)sizeof(K));
+  const bool wide = nc > 16 && E.nb > 512;
   if (nc <= 8)
     launch_mdot_rows<K, 8, false>(E, U, nc, w, 0, part, misc);
   else
     launch_mdot_rows<K, 16, false>(E, U, nc, w, 0, part, misc);
   if (wide) reduce_cols_kernel<<<nc, 256, 0, stream()>>>(E.nb, nc, 0, E.pstride, part, ptot, misc);
-  hh_dT_kernel<<<1, 256, 0, stream()>>>(wide ? 1 : E.nb, E.pstride, wide ? ptot : part, j, small, E.lay);
+  hh_dT_kernel<<<1, kSmallBS, 0, stream()>>>(wide ? 1 : E.nb, E.pstride, wide ? ptot : part, j, small, E.lay);
   // fused update + tail multi-dot while the per-thread reflector row fits
   // in registers (up to 16 columns; 32 in FP32)
   if (nc <= 16 || (sizeof(K) == 4 && nc <= 32)) {
@@ -838,15 +977,14 @@ int hh_step(HHEngine<K>& E, int j, bool write_q) {
       hh_update_mdot_kernel<K, 32><<<E.nb, kBS, 0, stream()>>>(E.n, E.ld, U, nc, w, j + 1, E.rpb,
                                                               small, E.lay, part, E.pstride);
   } else {
-    LACE_NC_DISPATCH(nc, (hh_update_kernel<K, NCB><<<nbv, kBS, 0, stream()>>>(E.n, E.ld, U, nc, small,
-                                                                              E.lay, w)));
+    hh_update_kernel<K><<<nbv, kBS, 0, stream()>>>(E.n, E.ld, U, nc, small, E.lay, w);
     launch_mdot_rows<K, 16, true>(E, U, nc, w, j + 1, part, misc);
   }
   if (wide) reduce_cols_kernel<<<nc + 1, 256, 0, stream()>>>(E.nb, nc, 1, E.pstride, part, ptot, misc);
-  hh_newcol_small_kernel<K><<<1, 256, 0, stream()>>>(wide ? 1 : E.nb, E.pstride, wide ? ptot : part, j,
+  hh_newcol_small_kernel<K><<<1, kSmallBS, 0, stream()>>>(wide ? 1 : E.nb, E.pstride, wide ? ptot : part, j,
                                                      E.n, E.ld, U, w, small, E.lay);
-  LACE_NC_DISPATCH(nc, (hh_newcol_vec_kernel<K, NCB><<<nbv, kBS, 0, stream()>>>(
-                           E.n, E.ld, U, j, w, small, E.lay, E.q.template as<K>(), write_q ? 1 : 0)));
+  hh_newcol_vec_kernel<K><<<nbv, kBS, 0, stream()>>>(E.n, E.ld, U, j, w, small, E.lay, E.q.template as<K>(),
+                                                     write_q ? 1 : 0);
   LACE_HIP(hipGetLastError());
   return DEV_SUCCESS;
 }
@@ -1052,7 +1190,7 @@ __global__ __launch_bounds__(256) void cgs_small_kernel(int nb, int pstride, con
   }
   if (threadIdx.x == 0) pre[1] = misc[MS_RTOL];
   const int cnt = j < lay.m ? j + 1 : 0;
-  finalize_partials(nb, cnt, true, pstride, partial, s);  // s[0..cnt), s[cnt] = ||W_j||^2
+  finalize_partials<256>(nb, cnt, true, pstride, partial, s);  // s[0..cnt), s[cnt] = ||W_j||^2
   __syncthreads();
   if (done) return;
   if (threadIdx.x == 0) {
@@ -1136,15 +1274,20 @@ template int cgs_step<double>(HHEngine<double>&, int, bool, double);
 
 // Helpers used by the solver for norms and casts.
 int norm2_sq_partials(int n, int rpb, const double* x, double* partial, int pstride, int nb) {
-  mdot_kernel<double, 8, true><<<nb, kBS, 0, stream()>>>(n, n, x, 0, x, 0, rpb, partial, pstride,
-                                                        nullptr);
+  // 16-byte words, all threads on the rows, where x allows (4096 to 200000
+  // rows: 19 -> 5 us)
+  if (rpb == 4 * kBS && reinterpret_cast<uintptr_t>(x) % 16 == 0)
+    mdot_rows_kernel<double, 8, true, 4><<<nb, kBS, 0, stream()>>>(n, n, x, 0, x, 0, rpb, 8, partial, pstride,
+                                                                   nullptr);
+  else
+    mdot_kernel<double, 8, true><<<nb, kBS, 0, stream()>>>(n, n, x, 0, x, 0, rpb, partial, pstride, nullptr);
   LACE_HIP(hipGetLastError());
   return DEV_SUCCESS;
 }
 
 __global__ __launch_bounds__(256) void sum_slot_kernel(int nb, int pstride, const double* partial, double* out) {
   __shared__ double v[1];
-  finalize_partials(nb, 0, true, pstride, partial, v);
+  finalize_partials<256>(nb, 0, true, pstride, partial, v);
   __syncthreads();
   if (threadIdx.x == 0) *out = v[0];
 }

@@ -322,7 +322,7 @@ struct Solver {
   std::unique_ptr<BlockEngine> beng;  // 32-right-hand-side solver, on first use
   MatlabLog mlog;  // progress lines of the drop-in FGMRES entry points
   DevBuf rbuf, partial, scal;
-  int nbn = 0, rpb = 4096, pstride = 4;
+  int nbn = 0, rpb = 1024, pstride = 4;
   double* host_scal = nullptr;
   ~Solver() {
     delete P;
