@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -138,6 +139,79 @@ __device__ __forceinline__ void stage_products(const int* __restrict__ col, cons
       }
     }
   }
+}
+
+// Row sums of a short block of rows [r0, r1), r1 - r0 <= 256 = blockDim.x:
+// thread t gets sum_k val[k] * x[col[k]] over row r0 + t, in entry order from
+// zero.  The block's entries are one contiguous range; each thread loads two
+// aligned groups of four (16-byte words), then gathers x for all eight, then
+// stages the products in LDS, so a block of up to kRowsCap entries waits for
+// memory three times whatever its rows' lengths: a matrix that fills the chip
+// with few blocks is bound by those waits, not by bytes.
+constexpr int kRowsCap = 2044;  // with the group cut off before the range: 512 groups
+
+// Rows of such a block: about kRowsCap entries, and fewer where the matrix
+// has too few rows for four blocks per CU.
+inline int rows_per_block(int n, long nnz) {
+  const long fit = nnz > 0 ? (long)((double)kRowsCap * n / nnz) : 256;
+  const long few = ((long)n / 1024 + 31) / 32 * 32;
+  return (int)std::max(32L, std::min(256L, std::min(fit / 32 * 32, std::max(64L, few))));
+}
+
+template <typename ACC, typename TV, typename TX>
+__device__ __forceinline__ ACC block_row_sum(const int* __restrict__ row, const int* __restrict__ col,
+                                             const TV* __restrict__ val, const TX* __restrict__ x, int r0, int r1,
+                                             ACC* prod) {
+#pragma clang fp contract(off)
+  const int i = r0 + (int)threadIdx.x;
+  int rs = 0, re = 0;
+  if (i < r1) rs = row[i], re = row[i + 1];
+  const int k0 = row[r0], k1 = row[r1];
+  ACC s = ACC(0);
+  for (int c0 = k0; c0 < k1; c0 += kRowsCap) {
+    const int end = min(c0 + kRowsCap, k1);
+    int c[2][4];
+    TV v[2][4];
+    TX g[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int k = (c0 & ~3) + 4 * ((int)threadIdx.x + 256 * u);
+      if (k + 3 < end) {
+        const int4 c4 = *reinterpret_cast<const int4*>(col + k);
+        c[u][0] = c4.x, c[u][1] = c4.y, c[u][2] = c4.z, c[u][3] = c4.w;
+        load4(val + k, v[u]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          c[u][e] = k + e < end ? col[k + e] : -1;
+          v[u][e] = k + e < end ? val[k + e] : TV(0);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) g[u][e] = c[u][e] >= 0 ? x[c[u][e]] : TX(0);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int k = (c0 & ~3) + 4 * ((int)threadIdx.x + 256 * u);
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (k + e >= c0 && k + e < end) prod[k + e - c0] = (ACC)v[u][e] * (ACC)g[u][e];
+    }
+    __syncthreads();
+    const int lo = max(rs, c0) - c0, hi = min(re, end) - c0;
+    for (int k = lo; k < hi; k += 4) {
+      ACC p[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) p[e] = k + e < hi ? prod[k + e] : ACC(0);
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (k + e < hi) s = s + p[e];
+    }
+    __syncthreads();
+  }
+  return s;
 }
 
 template <typename T>

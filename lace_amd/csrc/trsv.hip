@@ -1270,15 +1270,51 @@ __global__ void tri_diag_div_kernel(int n, const T* __restrict__ dval, const T* 
   if (i < n) y[i] = r[i] / dval[i];
 }
 
+// The same sweep on short blocks of rows (block_row_sum), the default; with
+// y2 and d2 given it also writes y2 = yout / d2, the first sweep of a following
+// solve.  Five sweeps of L and U on ragged meshes, against blocks of 256 R
+// rows: 1320 rows FP64 35 -> 25 us, 91000 rows FP64 43 -> 34 us, 148000 rows
+// FP32 59 -> 35 us, 2 10^6 rows FP32 272 -> 202 us and FP64 370 -> 302 us.
+template <typename T, bool UNIT>
+__global__ __launch_bounds__(256) void tri_jacobi_rows_kernel(
+    int n, int rpb, const int* __restrict__ srow, const int* __restrict__ scol, const T* __restrict__ sval,
+    const T* __restrict__ dval, const T* __restrict__ r, const T* __restrict__ yin, T* __restrict__ yout,
+    T* __restrict__ y2, const T* __restrict__ d2) {
+#pragma clang fp contract(off)
+  __shared__ T prod[kRowsCap];
+  const int r0 = xcd_block(blockIdx.x, gridDim.x) * rpb, r1 = min(r0 + rpb, n);
+  const int i = r0 + (int)threadIdx.x;
+  T rr = T(0), dg = T(1);
+  if (i < r1) {
+    rr = r[i];
+    if (!UNIT) dg = dval[i];
+  }
+  const T s = block_row_sum<T>(srow, scol, sval, yin, r0, r1, prod);
+  if (i < r1) {
+    const T y = UNIT ? rr - s : (rr - s) / dg;
+    yout[i] = y;
+    if (y2) y2[i] = y / d2[i];
+  }
+}
+
 template <typename T, bool UNIT, int R>
 static void launch_jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* yout) {
   tri_jacobi_strict_kernel<T, UNIT, R><<<ceil_div(P.n, JacCap<T, R>::rows), 256, 0, stream()>>>(
       P.n, P.srow.as<int>(), P.scol.as<int>(), P.sval.as<T>(), P.dval.as<T>(), r, yin, yout);
 }
 
+static bool jacobi_rows() { return get_option("stream_rows_per_thread", 0) == 0; }
+
+// y2, d2: with jacobi_rows only.
 template <typename T, bool UNIT>
-static void jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* yout) {
-  const int R = get_option("stream_rows_per_thread", sizeof(T) == 8 ? 1 : 2);
+static void jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* yout, T* y2, const T* d2) {
+  if (jacobi_rows()) {
+    const int rpb = rows_per_block(P.n, P.snnz);
+    tri_jacobi_rows_kernel<T, UNIT><<<ceil_div(P.n, rpb), 256, 0, stream()>>>(
+        P.n, rpb, P.srow.as<int>(), P.scol.as<int>(), P.sval.as<T>(), P.dval.as<T>(), r, yin, yout, y2, d2);
+    return;
+  }
+  const int R = get_option("stream_rows_per_thread", 0);
   if (R == 1) launch_jacobi_strict<T, UNIT, 1>(P, r, yin, yout);
   else if (R == 4) launch_jacobi_strict<T, UNIT, 4>(P, r, yin, yout);
   else launch_jacobi_strict<T, UNIT, 2>(P, r, yin, yout);
@@ -1465,7 +1501,7 @@ static int jacobi_sweep(const TriPlan& P, const T* val, const T* r, const T* yin
   if (!partial && yin && P.n > 0 && P.nnz <= 16LL * P.n) {
     const bool dia = strict && P.dia.nd > 0 && get_option("jacobi_dia", 1) != 0;
     const bool ell = !dia && strict && P.ew > 0 && get_option("jacobi_ell", 1) != 0;
-    const bool fuse = dia && y2 && d2;
+    const bool fuse = (dia || (strict && !ell && jacobi_rows())) && y2 && d2;
     // 16-bit words of the diagonal form where the factors are stored in 16
     // bits (four rows per thread; it needs n % 4 == 0 and aligned vectors)
     const bool d16 = dia && sizeof(T) == 4 && P.dia16_fmt != LACE_F32 && P.dia16_src == (const void*)val &&
@@ -1500,8 +1536,8 @@ static int jacobi_sweep(const TriPlan& P, const T* val, const T* r, const T* yin
     else if (dia) jacobi_dia<T, false>(P, r, yin, yout, fuse ? y2 : nullptr, d2, tr);
     else if (ell && P.unit_diag) jacobi_ell<T, true>(P, r, yin, yout);
     else if (ell) jacobi_ell<T, false>(P, r, yin, yout);
-    else if (strict && P.unit_diag) jacobi_strict<T, true>(P, r, yin, yout);
-    else if (strict) jacobi_strict<T, false>(P, r, yin, yout);
+    else if (strict && P.unit_diag) jacobi_strict<T, true>(P, r, yin, yout, fuse ? y2 : nullptr, d2);
+    else if (strict) jacobi_strict<T, false>(P, r, yin, yout, fuse ? y2 : nullptr, d2);
     else if (P.upper) jacobi_stream<T, true>(P, val, r, yin, yout);
     else jacobi_stream<T, false>(P, val, r, yin, yout);
     LACE_HIP(hipGetLastError());
@@ -1849,7 +1885,7 @@ static int apply_t(ParILU* P, lace_trsv_kind_t kind, int sweeps, int trans, cons
   }
   // For an odd sweep count the second solve's first sweep (tmp / diag,
   // written to z) rides on the first solve's last sweep when that runs on
-  // the diagonal form; z is then distinct from every buffer that sweep reads.
+  // the diagonal form or on blocks of rows; z is then distinct from every buffer that sweep reads.
   const bool fuse = first.unit_diag && !second.unit_diag && sweeps % 2 == 1 &&
                     second.strict_src == (const void*)v2 && (const void*)z != (const void*)r &&
                     get_option("jacobi_fuse", 1) != 0;
