@@ -162,16 +162,23 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream_sweep_kernel(
 // row, which precede it: those among the thread's positions and the four
 // before them (the previous lanes', shuffled in before any branch) come
 // from registers, only earlier ones (rows longer than the window, the
-// first lanes of a wave) from memory, in the same ascending order.
+// first lanes of a wave) from memory, in the same ascending order.  With
+// MATCH (patterns whose strict positions have matches of their own) the
+// block's positions and the 16 before them are in LDS, from where a row's own
+// values come; row j's values are gathered two matches at a time for all of a
+// thread's positions together, and registers are held to six blocks per CU
+// (one round of the chip up to 786000 positions): 91000-row mesh FP64 23.0 ->
+// 21.2 us, 148000-row mesh FP32 25.2 -> 21.4 us, of which 14 us are the
+// 70 MB it moves.
 template <typename T, bool STEP, bool MATCH, int P>
-__global__ __launch_bounds__(kSweepBS) void parilu_stream4_sweep_kernel(
+__global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_kernel(
     int np, const int* __restrict__ pmeta, const int* __restrict__ mptr,
     const int* __restrict__ mpairs, const T* __restrict__ AL, const T* __restrict__ AU,
     const T* __restrict__ VLin, const T* __restrict__ VUin, T* __restrict__ VLout,
     T* __restrict__ VUout, double* __restrict__ partial) {
 #pragma clang fp contract(off)
   static_assert(P == 2 || P == 4, "two or four positions per thread");
-  static_assert(P * sizeof(T) % 16 == 0, "16-byte words of P values");
+  constexpr int MB = 2;  // matches whose operands are loaded together
   constexpr int W = 4;  // positions of the window before the thread's first
   const int b = xcd_block(blockIdx.x, gridDim.x);
   const int p0 = (b * kSweepBS + (int)threadIdx.x) * P;
@@ -184,10 +191,10 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream4_sweep_kernel(
   // entry 0 and ignores it)
   if (full) {
     wload<int, P>(pmeta + p0, mv);
-    vload<T, P>(AL + p0, al);
-    vload<T, P>(AU + p0, au);
-    vload<T, P>(VLin + p0, lo);
-    vload<T, P>(VUin + p0, uo);
+    wload<T, P>(AL + p0, al);
+    wload<T, P>(AU + p0, au);
+    wload<T, P>(VLin + p0, lo);
+    wload<T, P>(VUin + p0, uo);
 #pragma unroll
     for (int e = 0; e < P; e++) ujj[e] = VUin[max(mv[e], 0)];
   } else {
@@ -214,6 +221,54 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream4_sweep_kernel(
     plo[k] = __shfl_up(lo[e], back);
     puo[k] = __shfl_up(uo[e], back);
   }
+  // a strict position's first MB matches: places in rows i and j, and row
+  // j's values (a place past the last match reads entry 0, which is not
+  // used).  Row i's values come from LDS, which holds the block's positions
+  // and the H before them.
+  constexpr int H = 16;
+  __shared__ T own[MATCH ? 2 : 1][MATCH ? kSweepBS * P + H : 1];
+  const int h0 = b * kSweepBS * P - H;
+  if (MATCH) {
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      own[0][H + (int)threadIdx.x * P + e] = lo[e];
+      own[MATCH][H + (int)threadIdx.x * P + e] = uo[e];
+    }
+    if (threadIdx.x < H && h0 >= 0) {
+      own[0][threadIdx.x] = VLin[h0 + threadIdx.x];
+      own[MATCH][threadIdx.x] = VUin[h0 + threadIdx.x];
+    }
+  }
+  int t0[P + 1];
+  int2 mq[P][MB];
+  T lc[P][MB], uc[P][MB];
+  if (MATCH && p0 < np) {
+#pragma unroll
+    for (int e = 0; e <= P; e++) t0[e] = mptr[min(p0 + e, np)];
+#pragma unroll
+    for (int e = 0; e < P; e++)
+#pragma unroll
+      for (int k = 0; k < MB; k++)
+        mq[e][k] = t0[e] + k < t0[e + 1] ? reinterpret_cast<const int2*>(mpairs)[t0[e] + k] : int2{0, 0};
+#pragma unroll
+    for (int e = 0; e < P; e++)
+#pragma unroll
+      for (int k = 0; k < MB; k++) {
+        uc[e][k] = VUin[mq[e][k].y];
+        lc[e][k] = VLin[mq[e][k].y];
+      }
+  }
+  if (MATCH) __syncthreads();
+  // l and u at position q of the row of position p >= q
+  const auto mine = [&](int q, T& l, T& u) {
+    if (q >= h0) {
+      l = own[0][q - h0];
+      u = own[MATCH][q - h0];
+    } else {
+      l = VLin[q];
+      u = VUin[q];
+    }
+  };
   double d2 = 0.0;
   if (p0 < np) {
 #pragma unroll
@@ -226,9 +281,20 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream4_sweep_kernel(
       } else if (m < 0) {
         const int i0 = -m - 1;
         T s = au[e];
-        for (int q = i0; q < min(p, p0 - W); q++) s = s - VLin[q] * VUin[q];
+        if (MATCH) {
+          for (int q0 = i0; q0 < p; q0 += MB) {
+            T lq[MB], uq[MB];
 #pragma unroll
-        for (int k = -W; k < e; k++) {
+            for (int k = 0; k < MB; k++) mine(min(q0 + k, p), lq[k], uq[k]);
+#pragma unroll
+            for (int k = 0; k < MB; k++)
+              if (q0 + k < p) s = s - lq[k] * uq[k];
+          }
+        } else {
+          for (int q = i0; q < min(p, p0 - W); q++) s = s - VLin[q] * VUin[q];
+        }
+#pragma unroll
+        for (int k = MATCH ? 0 : -W; k < (MATCH ? 0 : e); k++) {
           const int q = p0 + k;
           if (q >= i0) {
             T lq, uq;
@@ -257,10 +323,33 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream4_sweep_kernel(
       } else {
         T sL = al[e], sU = au[e];
         if (MATCH) {
-          for (int t = mptr[p]; t < mptr[p + 1]; t++) {
-            const int qa = mpairs[2 * t], qc = mpairs[2 * t + 1];
-            sL = sL - VLin[qa] * VUin[qc];
-            sU = sU - VLin[qc] * VUin[qa];
+#pragma unroll
+          for (int k = 0; k < MB; k++)
+            if (t0[e] + k < t0[e + 1]) {
+              T l, u;
+              mine(mq[e][k].x, l, u);
+              sL = sL - l * uc[e][k];
+              sU = sU - lc[e][k] * u;
+            }
+          for (int t = t0[e] + MB; t < t0[e + 1]; t += MB) {
+            int2 q[MB];
+            T u1[MB], l2[MB];
+#pragma unroll
+            for (int k = 0; k < MB; k++)
+              q[k] = t + k < t0[e + 1] ? reinterpret_cast<const int2*>(mpairs)[t + k] : int2{0, 0};
+#pragma unroll
+            for (int k = 0; k < MB; k++) {
+              u1[k] = VUin[q[k].y];
+              l2[k] = VLin[q[k].y];
+            }
+#pragma unroll
+            for (int k = 0; k < MB; k++)
+              if (t + k < t0[e + 1]) {
+                T l, u;
+                mine(q[k].x, l, u);
+                sL = sL - l * u1[k];
+                sU = sU - l2[k] * u;
+              }
           }
         }
         sU = sU - pu;
@@ -279,8 +368,8 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream4_sweep_kernel(
       }
     }
     if (full) {
-      vstore<T, P>(VLout + p0, lout);
-      vstore<T, P>(VUout + p0, uout);
+      wstore<T, P>(VLout + p0, lout);
+      wstore<T, P>(VUout + p0, uout);
     } else {
 #pragma unroll
       for (int e = 0; e < P; e++)
@@ -924,17 +1013,18 @@ static int sweep_t(ParILU* P, bool with_step) {
   // (128^3: FP32 38.8 us vs 43.7 us for one position per thread)
   if (stream4) {
     // four positions per thread in FP32, two in FP64 (one 16-byte word per
-    // array either way)
+    // array either way); two where strict positions have matches, whose
+    // operands take the registers
     constexpr int PP = sizeof(T) == 8 ? 2 : 4;
-    const int nb = ceil_div(P->nnzL, kSweepBS * PP);
+    const int nb = ceil_div(P->nnzL, kSweepBS * (P->strict_matches ? 2 : PP));
     auto go = [&](auto kern) {
       tr.launch(kern, dim3(nb), dim3(kSweepBS), P->nnzL, P->pmeta.as<int>(), P->mptr.as<int>(),
                 P->mpairs.as<int>(), P->AL.as<T>(), P->AU.as<T>(), P->lval[in].as<T>(),
                 P->uval[in].as<T>(), P->lval[out].as<T>(), P->uval[out].as<T>(), P->partial.as<double>());
     };
     if (P->strict_matches) {
-      if (with_step) go(parilu_stream4_sweep_kernel<T, true, true, PP>);
-      else go(parilu_stream4_sweep_kernel<T, false, true, PP>);
+      if (with_step) go(parilu_stream4_sweep_kernel<T, true, true, 2>);
+      else go(parilu_stream4_sweep_kernel<T, false, true, 2>);
     } else {
       if (with_step) go(parilu_stream4_sweep_kernel<T, true, false, PP>);
       else go(parilu_stream4_sweep_kernel<T, false, false, PP>);
