@@ -281,4 +281,10 @@ __device__ __forceinline__ TC dequant(TS q, float s) {
   }
 }
 
+// v as a 16-bit store with row scale s would return it.
+template <typename TS>
+__device__ __forceinline__ float round_stored(float v, float s) {
+  return dequant<float, TS>(quant<float, TS>(v, 1.0f / s), s);
+}
+
 }  // namespace lace

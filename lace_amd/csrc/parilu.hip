@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -170,12 +171,19 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream_sweep_kernel(
 // (one round of the chip up to 786000 positions): 91000-row mesh FP64 23.0 ->
 // 21.2 us, 148000-row mesh FP32 25.2 -> 21.4 us, of which 14 us are the
 // 70 MB it moves.
-template <typename T, bool STEP, bool MATCH, int P>
+//
+// With 16-bit storage (TS not T) the new values are rounded to 16 bits
+// relative to their row's scale before they are stored and compared, as
+// parilu_round16_kernel rounds them: l_ij by rs[prow], u_ji by rs[pcol] of
+// its position (100 x 77 x 53 BF16: 21 us a sweep for the two launches, 13 us
+// in one; reset 34 -> 17 us).
+template <typename T, typename TS, bool STEP, bool MATCH, int P>
 __global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_kernel(
     int np, const int* __restrict__ pmeta, const int* __restrict__ mptr,
     const int* __restrict__ mpairs, const T* __restrict__ AL, const T* __restrict__ AU,
     const T* __restrict__ VLin, const T* __restrict__ VUin, T* __restrict__ VLout,
-    T* __restrict__ VUout, double* __restrict__ partial) {
+    T* __restrict__ VUout, double* __restrict__ partial, const int* __restrict__ prow,
+    const int* __restrict__ pcol, const float* __restrict__ rs) {
 #pragma clang fp contract(off)
   static_assert(P == 2 || P == 4, "two or four positions per thread");
   constexpr int MB = 2;  // matches whose operands are loaded together
@@ -184,8 +192,29 @@ __global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_
   const int p0 = (b * kSweepBS + (int)threadIdx.x) * P;
   const int lane = threadIdx.x & 63;
   const bool full = p0 + P - 1 < np;
+  constexpr bool S16 = !std::is_same<T, TS>::value;
   int mv[P];
   T al[P], au[P], lo[P], uo[P], lout[P], uout[P], ujj[P];
+  float sl[P], su[P];  // row scales of l and u
+  if constexpr (S16) {
+    int ri[P], ci[P];
+    if (full) {
+      wload<int, P>(prow + p0, ri);
+      wload<int, P>(pcol + p0, ci);
+    } else {
+#pragma unroll
+      for (int e = 0; e < P; e++) {
+        const int p = max(0, min(p0 + e, np - 1));
+        ri[e] = prow[p];
+        ci[e] = pcol[p];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      sl[e] = rs[ri[e]];
+      su[e] = rs[ci[e]];
+    }
+  }
   // u_jj of each strict position is gathered as soon as pmeta is in, in
   // the branch that loads it (every index valid: a diagonal position reads
   // entry 0 and ignores it)
@@ -314,6 +343,7 @@ __global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_
         }
         s = s - pu;
         s = s + pu;
+        if constexpr (S16) s = round_stored<TS>(s, su[e]);
         uout[e] = s;
         lout[e] = lo[e];
         if (STEP) {
@@ -354,11 +384,13 @@ __global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_
         }
         sU = sU - pu;
         sU = sU + pu;
+        if constexpr (S16) sU = round_stored<TS>(sU, su[e]);
         uout[e] = sU;
         const T pl = lo[e] * ujj[e];
         sL = sL - pl;
         sL = sL + pl;
-        const T t = sL / ujj[e];
+        T t = sL / ujj[e];
+        if constexpr (S16) t = round_stored<TS>(t, sl[e]);
         lout[e] = t;
         if (STEP) {
           const double d1 = (double)uo[e] - (double)sU;
@@ -438,14 +470,19 @@ __global__ void parilu_scatter_sym_kernel(int nnz, const int* __restrict__ dst, 
 // positions coincide (L in CSR, U in CSC), AL holds a_ij and AU a_ji at the
 // position of (i, j), so L0 = AL with a unit diagonal and U0 = AU; reads and
 // writes are coalesced (the scatter from A's CSR order is not).
-template <typename T>
+template <typename T, typename TS>
 __global__ void parilu_reset_sym_kernel(int np, const int* __restrict__ pmeta, const T* __restrict__ AL,
                                         const T* __restrict__ AU, T* __restrict__ L0, T* __restrict__ L1,
-                                        T* __restrict__ U0, T* __restrict__ U1) {
+                                        T* __restrict__ U0, T* __restrict__ U1, const int* __restrict__ prow,
+                                        const int* __restrict__ pcol, const float* __restrict__ rs) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
-  const T l = pmeta[p] < 0 ? T(1) : AL[p];
-  const T u = AU[p];
+  T l = AL[p], u = AU[p];
+  if constexpr (!std::is_same<T, TS>::value) {
+    l = round_stored<TS>(l, rs[prow[p]]);
+    u = round_stored<TS>(u, rs[pcol[p]]);
+  }
+  if (pmeta[p] < 0) l = T(1);
   L0[p] = l;
   L1[p] = l;
   U0[p] = u;
@@ -923,16 +960,19 @@ static int build_pattern(const data_d_matrix* A, ParILU* P, ParILUUse use) {
 
 int ParILU::reset() {
   const int nb = ceil_div(nnz, 256);
-  if (sym && pmeta.p && AL.p && AU.p) {
+  const bool at_reset = sym && pmeta.p && AL.p && AU.p;  // that kernel rounds
+  if (at_reset) {
     const int nbl = ceil_div(nnzL, 256);
-    if (prec == LACE_F64)
-      parilu_reset_sym_kernel<double><<<nbl, 256, 0, stream()>>>(
-          nnzL, pmeta.as<int>(), AL.as<double>(), AU.as<double>(), lval[0].as<double>(), lval[1].as<double>(),
-          uval[0].as<double>(), uval[1].as<double>());
-    else
-      parilu_reset_sym_kernel<float><<<nbl, 256, 0, stream()>>>(
-          nnzL, pmeta.as<int>(), AL.as<float>(), AU.as<float>(), lval[0].as<float>(), lval[1].as<float>(),
-          uval[0].as<float>(), uval[1].as<float>());
+    const auto go = [&](auto kern, auto zero) {
+      using T = decltype(zero);
+      kern<<<nbl, 256, 0, stream()>>>(nnzL, pmeta.as<int>(), AL.as<T>(), AU.as<T>(), lval[0].as<T>(),
+                                      lval[1].as<T>(), uval[0].as<T>(), uval[1].as<T>(), prow.as<int>(),
+                                      lcol.as<int>(), rs.as<float>());
+    };
+    if (prec == LACE_F64) go(parilu_reset_sym_kernel<double, double>, 0.0);
+    else if (prec == LACE_F32) go(parilu_reset_sym_kernel<float, float>, 0.0f);
+    else if (prec == LACE_BF16) go(parilu_reset_sym_kernel<float, uint16_t>, 0.0f);
+    else go(parilu_reset_sym_kernel<float, _Float16>, 0.0f);
   } else if (prec == LACE_F64) {
     parilu_reset_kernel<double><<<nb, 256, 0, stream()>>>(nnz, dst.as<int>(), aval.as<double>(),
                                                           lval[0].as<double>(), lval[1].as<double>(),
@@ -949,7 +989,7 @@ int ParILU::reset() {
   LACE_HIP(hipGetLastError());
   cur = 0;
   csr_dirty = true;
-  if (s16()) LACE_TRY(round16(true, false));
+  if (s16() && !at_reset) LACE_TRY(round16(true, false));
   return DEV_SUCCESS;
 }
 
@@ -1020,14 +1060,25 @@ static int sweep_t(ParILU* P, bool with_step) {
     auto go = [&](auto kern) {
       tr.launch(kern, dim3(nb), dim3(kSweepBS), P->nnzL, P->pmeta.as<int>(), P->mptr.as<int>(),
                 P->mpairs.as<int>(), P->AL.as<T>(), P->AU.as<T>(), P->lval[in].as<T>(),
-                P->uval[in].as<T>(), P->lval[out].as<T>(), P->uval[out].as<T>(), P->partial.as<double>());
+                P->uval[in].as<T>(), P->lval[out].as<T>(), P->uval[out].as<T>(), P->partial.as<double>(),
+                P->prow.as<int>(), P->lcol.as<int>(), P->rs.as<float>());
     };
-    if (P->strict_matches) {
-      if (with_step) go(parilu_stream4_sweep_kernel<T, true, true, 2>);
-      else go(parilu_stream4_sweep_kernel<T, false, true, 2>);
+    const auto stored = [&](auto ts) {
+      using TS = decltype(ts);
+      if (P->strict_matches) {
+        if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, true, 2>);
+        else go(parilu_stream4_sweep_kernel<T, TS, false, true, 2>);
+      } else {
+        if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, false, PP>);
+        else go(parilu_stream4_sweep_kernel<T, TS, false, false, PP>);
+      }
+    };
+    if constexpr (sizeof(T) == 8) {
+      stored(0.0);
     } else {
-      if (with_step) go(parilu_stream4_sweep_kernel<T, true, false, PP>);
-      else go(parilu_stream4_sweep_kernel<T, false, false, PP>);
+      if (P->prec == LACE_BF16) stored(uint16_t(0));
+      else if (P->prec == LACE_F16) stored(_Float16(0));
+      else stored(0.0f);
     }
     LACE_HIP(hipGetLastError());
     P->last_nb = nb;
@@ -1138,6 +1189,8 @@ int ParILU::round16(bool both_buffers, bool with_step) {
 int ParILU::sweep(bool with_step) {
   if (prec == LACE_F64) return sweep_t<double>(this, with_step);
   if (!s16()) return sweep_t<float>(this, with_step);
+  // the streaming kernel rounds to 16-bit storage itself
+  if (sym && (variant == 0 || variant == 5)) return sweep_t<float>(this, with_step);
   // FP32 sweep, then the rounding to 16-bit storage (which forms the step
   // from the stored values)
   LACE_TRY(sweep_t<float>(this, false));

@@ -137,7 +137,7 @@ struct TriPlan {
   int copy_ring(const TriPlan& o);
   int refresh_strict(const void* val, size_t elem_size);
   int ensure_forms(unsigned forms);
-  // 16-bit diagonal form (fmt BF16 or F16) from the current FP32 forms,
+  // 16-bit diagonal form (fmt BF16 or F16) from the value array strict_src,
   // whose values are already 16-bit values times the row scales rs.
   int refresh_dia16(lace_prec_t fmt, const float* rs);
 };
@@ -259,7 +259,7 @@ struct ParILU {
   // (lval_t) on a first transposed solve, and the off-diagonal forms the
   // Jacobi sweeps will read.
   bool lval_t_dirty = true;
-  int prepare(lace_trsv_kind_t kind, int trans, bool block);
+  int prepare(lace_trsv_kind_t kind, int trans, bool block, int sweeps = 0);
   // z = M^{-1} r (trans = 0) or M^{-T} r (trans = 1); r and z in the
   // factor precision (double for F64, float otherwise).
   int apply(lace_trsv_kind_t kind, int sweeps, int trans, const void* r, void* z);

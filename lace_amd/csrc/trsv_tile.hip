@@ -248,11 +248,20 @@ static void tile_dispatch(const TriPlan& P, const TS* dia, const TS* dval, const
 #undef LACE_TILE_CASE
 }
 
+bool jacobi_tile16(const TriPlan& P) {
+  return P.grid[0] > 0 && P.dia16_fmt != LACE_F32 && P.dia16_src != nullptr && P.dia16_src == P.strict_src &&
+         P.upper != P.unit_diag && (double)P.n * sizeof(float) < 2147483648.0 &&
+         get_option("jacobi_dia16", 1) != 0 && get_option("jacobi_dia", 1) != 0 &&
+         get_option("jacobi_dia_vec", 1) != 0;
+}
+
 template <typename T>
 bool jacobi_tile_ready(const TriPlan& P, const T* val, int sweeps) {
-  return sweeps >= 2 && P.grid[0] > 0 && P.strict_src == (const void*)val && !(P.stale & TriPlan::kFormDia) &&
-         (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) && (double)P.n * sizeof(T) < 2147483648.0 &&
-         get_option("jacobi_dia", 1) != 0 && get_option("jacobi_dia_vec", 1) != 0;
+  if (sweeps < 2 || P.strict_src != (const void*)val) return false;
+  if (sizeof(T) == 4 && jacobi_tile16(P)) return true;
+  return P.grid[0] > 0 && !(P.stale & TriPlan::kFormDia) && (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) &&
+         (double)P.n * sizeof(T) < 2147483648.0 && get_option("jacobi_dia", 1) != 0 &&
+         get_option("jacobi_dia_vec", 1) != 0;
 }
 
 template <typename T>
@@ -260,8 +269,7 @@ int jacobi_tile(const TriPlan& P, const T* r, const T* yin, T* yout, int c) {
   constexpr int W = 16 / (int)sizeof(T);
   const auto al16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
   const bool vec = P.grid[0] % W == 0 && al16(r) && al16(yin) && al16(yout);
-  const bool d16 = sizeof(T) == 4 && P.dia16_fmt != LACE_F32 && P.dia16_src == P.strict_src &&
-                   !(P.upper ? P.unit_diag : !P.unit_diag) && get_option("jacobi_dia16", 1) != 0;
+  const bool d16 = sizeof(T) == 4 && jacobi_tile16(P);
   const double es = sizeof(T), n = P.n, fs = d16 ? 2.0 : es;
   TimedRegion tr(P.upper ? "trsv_jacobi_sweep_upper" : "trsv_jacobi_sweep_lower", 0.0,
                  (P.dia.nd + (P.unit_diag ? 0 : 1)) * fs * n + (d16 ? n : 0.0) + (yin ? 3.0 : 2.0) * es * n, true);
