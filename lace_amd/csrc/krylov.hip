@@ -1162,7 +1162,7 @@ __device__ bool cgs_close_column(double* small, SmallLayout lay, int jc, double 
 // Step j's small part (j = m: the closing of column m - 1 only).  The state
 // the closing of column j - 1 reads is staged in LDS by every lane while
 // the partials are summed.
-__global__ __launch_bounds__(256) void cgs_small_kernel(int nb, int pstride, const double* partial, int j,
+__global__ __launch_bounds__(kSmallBS) void cgs_small_kernel(int nb, int pstride, const double* partial, int j,
                                                         double* small, SmallLayout lay, int set_rtol,
                                                         double rtol_rel) {
   double* misc = small + lay.misc();
@@ -1175,14 +1175,14 @@ __global__ __launch_bounds__(256) void cgs_small_kernel(int nb, int pstride, con
   __shared__ int fin;
   double* R = small + lay.R();
   double* sc = small + lay.T();  // 1 / ||W_k||, staged in scs
-  for (int k = threadIdx.x; k < j; k += 256) scs[k] = sc[k];
+  for (int k = threadIdx.x; k < j; k += kSmallBS) scs[k] = sc[k];
   const int ldR = lay.m + 1;
   const int jc = j - 1;
   if (j >= 1) {
     const double* cs = small + lay.cs();
     const double* sn = small + lay.sn();
-    for (int k = threadIdx.x; k <= jc; k += 256) hs[k] = R[k + (size_t)jc * ldR];
-    for (int k = threadIdx.x; k < jc; k += 256) {
+    for (int k = threadIdx.x; k <= jc; k += kSmallBS) hs[k] = R[k + (size_t)jc * ldR];
+    for (int k = threadIdx.x; k < jc; k += kSmallBS) {
       css[k] = cs[k];
       sns[k] = sn[k];
     }
@@ -1190,7 +1190,7 @@ __global__ __launch_bounds__(256) void cgs_small_kernel(int nb, int pstride, con
   }
   if (threadIdx.x == 0) pre[1] = misc[MS_RTOL];
   const int cnt = j < lay.m ? j + 1 : 0;
-  finalize_partials<256>(nb, cnt, true, pstride, partial, s);  // s[0..cnt), s[cnt] = ||W_j||^2
+  finalize_partials<kSmallBS>(nb, cnt, true, pstride, partial, s);  // s[0..cnt), s[cnt] = ||W_j||^2
   __syncthreads();
   if (done) return;
   if (threadIdx.x == 0) {
@@ -1213,12 +1213,12 @@ __global__ __launch_bounds__(256) void cgs_small_kernel(int nb, int pstride, con
   }
   __syncthreads();
   if (j >= 1)
-    for (int k = threadIdx.x; k <= jc; k += 256) R[k + (size_t)jc * ldR] = hs[k];
+    for (int k = threadIdx.x; k <= jc; k += kSmallBS) R[k + (size_t)jc * ldR] = hs[k];
   if (j >= lay.m || fin) return;
   // column j: h_kj = s_k (W_k . w) into R's column (rotated when it closes)
   // and the update's coefficients d_k = h_kj s_k
   double* d = small + lay.d();
-  for (int k = threadIdx.x; k <= j; k += 256) {
+  for (int k = threadIdx.x; k <= j; k += kSmallBS) {
     const double h = scs[k] * s[k];
     R[k + (size_t)j * ldR] = h;
     d[k] = h * scs[k];
@@ -1259,10 +1259,10 @@ int cgs_step(HHEngine<K>& E, int j, bool last, double rtol_rel) {
     launch_mdot_rows<K, 8, false>(E, U, nc, w, 0, part, misc);
   else
     launch_mdot_rows<K, 16, false>(E, U, nc, w, 0, part, misc);
-  cgs_small_kernel<<<1, 256, 0, stream()>>>(E.nb, E.pstride, part, j, small, E.lay, 1, rtol_rel);
+  cgs_small_kernel<<<1, kSmallBS, 0, stream()>>>(E.nb, E.pstride, part, j, small, E.lay, 1, rtol_rel);
   LACE_NC_DISPATCH(nc, (cgs_update_kernel<K, NCB><<<E.nb, kBS, 0, stream()>>>(
                            E.n, E.ld, U, nc, w, last ? 0 : 1, E.rpb, small, E.lay, part, E.pstride)));
-  if (last) cgs_small_kernel<<<1, 256, 0, stream()>>>(E.nb, E.pstride, part, E.m, small, E.lay, 1, rtol_rel);
+  if (last) cgs_small_kernel<<<1, kSmallBS, 0, stream()>>>(E.nb, E.pstride, part, E.m, small, E.lay, 1, rtol_rel);
   LACE_HIP(hipGetLastError());
   return DEV_SUCCESS;
 }
