@@ -122,7 +122,13 @@ struct TriPlan {
   int rgroups = 0;  // groups of four a row takes at most
   int rspan = 0;
   size_t rslots = 0;
-  DevBuf rdesc, rperm, rslot, ridx;
+  DevBuf rform;  // rdesc, rperm, rslot, each row's place in level order, ridx
+  const unsigned* rdesc() const { return rform.as<unsigned>(); }
+  int* rperm() const { return rform.as<int>() + 2 * (size_t)rchunks; }
+  int* rslot() const { return rperm() + 64 * (size_t)rchunks; }
+  int* rplace() const { return rslot() + (n + 1) / 2 * 2; }
+  unsigned short* ridx() const { return reinterpret_cast<unsigned short*>(rplace() + (n + 1) / 2 * 2); }
+  size_t rform_words() const { return 66 * (size_t)rchunks + 2 * (size_t)((n + 1) / 2 * 2); }  // before ridx
   mutable DevBuf rval, rdiag, rrhs, rsol;
   mutable const void* rval_src = nullptr;
   static constexpr unsigned kFormStrict = 1, kFormDiag = 2, kFormEll = 4, kFormDia = 8, kFormAll = 15;

@@ -14,7 +14,6 @@
 // by its remainder was slower than dividing (75 against 66 us on 64 x 64: the
 // exponent test and its branch cost what the division's steps do).
 #include <algorithm>
-#include <utility>
 
 #include "common.hpp"
 #include "device.hpp"
@@ -142,8 +141,12 @@ int TriPlan::build_ring(const int* row_, const int* col_, const int* perm_h, con
   for (int l = 0; l < nlev; l++) chunks += (lptr[l + 1] - lptr[l] + 63) / 64;
   const int all = (int)padded(chunks);
   if (all > kRingDescs) return DEV_SUCCESS;
-  std::vector<uint2> desc(all);
-  std::vector<int> rp((size_t)all * 64, -1), slot(n);
+  rchunks = all;
+  std::vector<int> form(rform_words(), -1);
+  uint2* desc = reinterpret_cast<uint2*>(form.data());
+  int* rp = form.data() + 2 * (size_t)all;
+  int* slot = rp + 64 * (size_t)all;
+  std::copy(pos.begin(), pos.end(), slot + (n + 1) / 2 * 2);
   int c = 0, groups = 0, gmax = 1;
   for (int l = 0; l < nlev; l++)
     for (int p0 = lptr[l]; p0 < lptr[l + 1]; p0 += 64, c++) {
@@ -162,22 +165,19 @@ int TriPlan::build_ring(const int* row_, const int* col_, const int* perm_h, con
     desc[c].x = (unsigned)groups << 11;
     desc[c].y = (unsigned)(nlev - 1) << 15;
   }
-  DevBuf dpos_;
-  LACE_TRY(upload(dpos_, pos.data(), sizeof(int) * pos.size()));
-  LACE_TRY(upload(rdesc, desc.data(), sizeof(uint2) * desc.size()));
-  LACE_TRY(upload(rperm, rp.data(), sizeof(int) * rp.size()));
-  LACE_TRY(upload(rslot, slot.data(), sizeof(int) * slot.size()));
   // one more group: where a chunk without operands points
   rslots = ((size_t)groups + 1) * 256;
-  LACE_TRY(ridx.alloc(sizeof(uint16_t) * rslots));
-  ring_index_kernel<<<all + 1, 64, 0, stream()>>>(all, rdesc.as<uint2>(), rperm.as<int>(), row.as<int>(),
-                                                  col.as<int>(), dpos_.as<int>(), upper, groups,
-                                                  ridx.as<uint16_t>());
+  const size_t words = rform_words();
+  rchunks = 0;  // until the form is there
+  LACE_TRY(rform.alloc(sizeof(int) * words + sizeof(uint16_t) * rslots));
+  LACE_HIP(hipMemcpyAsync(rform.p, form.data(), sizeof(int) * words, hipMemcpyHostToDevice, stream()));
+  LACE_HIP(hipStreamSynchronize(stream()));  // form is released on return
+  rchunks = all;
+  ring_index_kernel<<<all + 1, 64, 0, stream()>>>(all, reinterpret_cast<const uint2*>(rdesc()), rperm(),
+                                                  row.as<int>(), col.as<int>(), rplace(), upper, groups, ridx());
   LACE_HIP(hipGetLastError());
-  LACE_HIP(hipStreamSynchronize(stream()));  // dpos_ is released on return
   rgroups = gmax;
   rspan = span;
-  rchunks = all;
   return DEV_SUCCESS;
 }
 
@@ -200,12 +200,8 @@ int TriPlan::copy_ring(const TriPlan& o) {
   rval_src = nullptr;
   rchunks = 0;
   if (o.rchunks == 0) return DEV_SUCCESS;
-  const std::pair<DevBuf*, const DevBuf*> bufs[] = {
-      {&rdesc, &o.rdesc}, {&rperm, &o.rperm}, {&rslot, &o.rslot}, {&ridx, &o.ridx}};
-  for (const auto& b : bufs) {
-    LACE_TRY(b.first->alloc(b.second->bytes));
-    LACE_HIP(hipMemcpyAsync(b.first->p, b.second->p, b.second->bytes, hipMemcpyDeviceToDevice, stream()));
-  }
+  LACE_TRY(rform.alloc(o.rform.bytes));
+  LACE_HIP(hipMemcpyAsync(rform.p, o.rform.p, o.rform.bytes, hipMemcpyDeviceToDevice, stream()));
   rslots = o.rslots;
   rgroups = o.rgroups;
   rspan = o.rspan;
@@ -391,8 +387,8 @@ static int ring_launch(const TriPlan& P, const T* rhs, T* out) {
     set = true;
   }
   tri_ring_kernel<T, NG, W, DIRECT><<<1, W * 64, lds, stream()>>>(
-      P.nlev, P.rchunks, P.rdesc.as<uint2>(), P.rval.as<T>(), P.ridx.as<ushort4>(), rhs, P.rdiag.as<T>(),
-      P.rperm.as<int>(), out);
+      P.nlev, P.rchunks, reinterpret_cast<const uint2*>(P.rdesc()), P.rval.as<T>(), reinterpret_cast<const ushort4*>(P.ridx()), rhs, P.rdiag.as<T>(),
+      P.rperm(), out);
   LACE_HIP(hipGetLastError());
   return DEV_SUCCESS;
 }
@@ -429,7 +425,7 @@ static int ring_values(const TriPlan& P, const T* val) {
   if (P.rval.bytes < sizeof(T) * P.rslots) LACE_TRY(P.rval.alloc(sizeof(T) * P.rslots));
   for (DevBuf* b : {&P.rdiag, &P.rrhs, &P.rsol})
     if (b->bytes < sizeof(T) * rows) LACE_TRY(b->alloc(sizeof(T) * rows));
-  ring_gather_kernel<T><<<P.rchunks + 1, 64, 0, stream()>>>(P.rchunks, P.rdesc.as<uint2>(), P.rperm.as<int>(),
+  ring_gather_kernel<T><<<P.rchunks + 1, 64, 0, stream()>>>(P.rchunks, reinterpret_cast<const uint2*>(P.rdesc()), P.rperm(),
                                                             P.row.as<int>(), P.upper, P.rslots, val,
                                                             P.rval.as<T>(), P.rdiag.as<T>());
   LACE_HIP(hipGetLastError());
@@ -438,8 +434,8 @@ static int ring_values(const TriPlan& P, const T* val) {
 }
 
 template <typename T>
-static int ring_move(int m, const DevBuf& map, const int* map2, const T* in, T* out) {
-  ring_move_kernel<T><<<ceil_div(m, 256), 256, 0, stream()>>>(m, map.as<int>(), map2, in, out);
+static int ring_move(int m, const int* map, const int* map2, const T* in, T* out) {
+  ring_move_kernel<T><<<ceil_div(m, 256), 256, 0, stream()>>>(m, map, map2, in, out);
   LACE_HIP(hipGetLastError());
   return DEV_SUCCESS;
 }
@@ -449,20 +445,20 @@ int tri_solve_ring(const TriPlan& P, const T* val, const T* r, T* y) {
   LACE_REQUIRE((const void*)r != (const void*)y, DEV_ERR_ILLEGAL_VALUE, "exact solve needs distinct r and y");
   LACE_TRY(ring_values<T>(P, val));
   if (ring_direct(P)) return ring_solve<T, true>(P, r, y);
-  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm, nullptr, r, P.rrhs.as<T>()));
+  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm(), nullptr, r, P.rrhs.as<T>()));
   LACE_TRY((ring_solve<T, false>(P, P.rrhs.as<T>(), P.rsol.as<T>())));
-  return ring_move<T>(P.n, P.rslot, nullptr, P.rsol.as<T>(), y);
+  return ring_move<T>(P.n, P.rslot(), nullptr, P.rsol.as<T>(), y);
 }
 
 template <typename T>
 int tri_solve_ring2(const TriPlan& P, const T* val, const TriPlan& Q, const T* val2, const T* r, T* y) {
   LACE_TRY(ring_values<T>(P, val));
   LACE_TRY(ring_values<T>(Q, val2));
-  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm, nullptr, r, P.rrhs.as<T>()));
+  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm(), nullptr, r, P.rrhs.as<T>()));
   LACE_TRY((ring_solve<T, false>(P, P.rrhs.as<T>(), P.rsol.as<T>())));
-  LACE_TRY(ring_move<T>(Q.rchunks * 64, Q.rperm, P.rslot.as<int>(), P.rsol.as<T>(), Q.rrhs.as<T>()));
+  LACE_TRY(ring_move<T>(Q.rchunks * 64, Q.rperm(), P.rslot(), P.rsol.as<T>(), Q.rrhs.as<T>()));
   LACE_TRY((ring_solve<T, false>(Q, Q.rrhs.as<T>(), Q.rsol.as<T>())));
-  return ring_move<T>(Q.n, Q.rslot, nullptr, Q.rsol.as<T>(), y);
+  return ring_move<T>(Q.n, Q.rslot(), nullptr, Q.rsol.as<T>(), y);
 }
 
 template <typename T>
