@@ -46,6 +46,38 @@ __device__ __forceinline__ T block_sum(T v, T* smem) {
   return r;
 }
 
+// Workgroup barrier that orders LDS only: global loads issued ahead stay in
+// flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// q[w] = a[w] / d, correctly rounded, through rd = 1 / (double)d where a
+// divisor is used several times.  A quotient of two floats is at least 2^-49
+// of itself away from every midpoint between normal floats (24-bit numbers a,
+// d and a 25-bit midpoint m: a - m d is a nonzero multiple of its last place),
+// and a * rd is within 2^-52 of it, so narrowing rounds as the division does; a
+// quotient below the normal range may be a midpoint, so a wave that has one
+// (or a zero, in a lane that counts) divides.  FP64 products run at the rate of FP32 ones here, and the IEEE
+// division's ten instructions do not fit under the loads of a kernel that
+// divides in every sweep (32-column sweeps of U on 80 x 72 x 64: 114 -> 83 us;
+// with the test on each quotient instead of the least of four, 99 us).
+__device__ __forceinline__ void quot(const float (&a)[4], float d, double rd, bool counts, float (&q)[4]) {
+  float t[4];
+#pragma unroll
+  for (int w = 0; w < 4; w++) t[w] = (float)((double)a[w] * rd);
+  // (a minimum passes over NaNs, which need no division)
+  const float least = fminf(fminf(fabsf(t[0]), fabsf(t[1])), fminf(fabsf(t[2]), fabsf(t[3])));
+  if (__any(counts && least < 1.17549435e-38f)) {
+#pragma unroll
+    for (int w = 0; w < 4; w++) t[w] = a[w] / d;
+  }
+#pragma unroll
+  for (int w = 0; w < 4; w++) q[w] = t[w];
+}
+
 // Four consecutive values from a 4-element-aligned address.
 __device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
   const float4 t = *reinterpret_cast<const float4*>(p);

@@ -587,6 +587,186 @@ static int jacobi32_pair(const TriPlan& P, const T* r, const T* yin, T* yout) {
   return DEV_SUCCESS;
 }
 
+// Up to kMarchC coupled sweeps in one launch on the factors of a 7-point
+// stencil (TriPlan::grid), FP32.  A workgroup takes a tile of the grid's xy
+// plane, widened by the sweeps' reach on the side the factor reads from, eight
+// of the 32 columns (two lanes a point; the workgroups of the other columns run
+// beside it on the same XCD and share its cache lines) and a run of planes.  It walks the planes in the direction of the dependencies: sweep s at
+// a plane needs sweep s - 1 at that plane (the x and y neighbours through LDS)
+// and at the plane before (in registers), so each plane's values, r and the
+// last iterate pass through once for all sweeps; the next plane's loads are
+// issued before this plane's sweeps.  A run starts c planes early, since sweep
+// s is right from the s-th plane on, as it is from the s-th point of the
+// widened tile on.  Points outside the grid hold zeros.  Each row's sum runs in
+// CSR order: bit-identical to one-sweep launches.  Five sweeps on 80 x 72 x 64:
+// L 76 us (two launches of pairs) -> 62 us, U 99 us (its first sweep a launch
+// of its own) -> 83 us.  What bounds it is arithmetic (29 us of VALU for L) and
+// the address rate of 32-byte pieces of rows (four columns a workgroup: 73 us
+// for L); wider pieces leave smaller tiles and more halo.
+constexpr int kMarchC = 4;
+constexpr int kMarchBS = 1024;
+constexpr int kMarchLP = 2;                   // lanes a point
+constexpr int kMarchCG = 32 / (4 * kMarchLP);  // column groups
+struct MarchShape {
+  int nx, ny, nz, n;
+  int bx, by, bz;  // tile core and planes per run
+  int ex;          // widened tile's line
+  int pts;         // points of the widened tile
+  int kx, ky, kz;  // tiles and runs
+  int c;           // coupled sweeps
+  unsigned mx;     // 2^20 / ex, rounded up
+};
+
+template <bool UPPER, bool UNIT>
+__global__ __launch_bounds__(kMarchBS) void jacobi32_march_kernel(MarchShape g, const float* __restrict__ dia,
+                                                                  const float* __restrict__ dval,
+                                                                  const float* __restrict__ r,
+                                                                  const float* __restrict__ yin,
+                                                                  float* __restrict__ yout) {
+#pragma clang fp contract(off)
+  extern __shared__ float4 img[];  // [sweep][point][lane]
+  constexpr int LP = kMarchLP;
+  const int lane = threadIdx.x, t = lane / LP;
+  int wg = xcd_block(blockIdx.x, gridDim.x);
+  const int c0 = (wg % kMarchCG) * 4 * LP + lane % LP * 4;
+  wg /= kMarchCG;
+  const int tx = wg % g.kx, tyz = wg / g.kx, ty = tyz % g.ky, tz = tyz / g.ky;
+  // coordinates counted in the direction of the dependencies
+  const int uy = (int)(((unsigned)t * g.mx) >> 20), ux = t - uy * g.ex;
+  const int x = tx * g.bx - g.c + ux, y = ty * g.by - g.c + uy;
+  const bool in = t < g.pts && x >= 0 && x < g.nx && y >= 0 && y < g.ny;
+  const bool core = in && ux >= g.c && uy >= g.c && ux < g.c + g.bx && uy < g.c + g.by;
+  const int z0 = tz * g.bz, z1 = min(z0 + g.bz, g.nz), zs = max(0, z0 - g.c);
+  const int line = (UPPER ? g.nx - 1 - x : x) + g.nx * (UPPER ? g.ny - 1 - y : y);
+  const int plane = g.nx * g.ny;
+  struct Point {
+    float v[3], d, rr[4], y0[4];
+  };
+  const auto load = [&](Point& p, int z) {
+    p.v[0] = p.v[1] = p.v[2] = 0.0f;
+    p.d = 1.0f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) p.rr[w] = p.y0[w] = 0.0f;
+    if (in && z < z1) {
+      const unsigned i = (unsigned)(line + plane * (UPPER ? g.nz - 1 - z : z));
+#pragma unroll
+      for (int q = 0; q < 3; q++) p.v[q] = dia[(size_t)q * g.n + i];
+      if (!UNIT) p.d = dval[i];
+      vload<float, 4>(r + (size_t)i * 32 + c0, p.rr);
+      if (yin) vload<float, 4>(yin + (size_t)i * 32 + c0, p.y0);
+    }
+  };
+  float prev[kMarchC][4];  // sweep s at the plane before
+#pragma unroll
+  for (int s = 0; s < kMarchC; s++)
+#pragma unroll
+    for (int w = 0; w < 4; w++) prev[s][w] = 0.0f;
+  Point a, b;
+  load(a, zs);
+  // one plane's sweeps, while the next plane's operands come in
+  const auto step = [&](const Point& p, int z) {
+    float yv[4];
+    const double rd = UNIT ? 1.0 : 1.0 / (double)p.d;
+#pragma unroll
+    for (int w = 0; w < 4; w++) yv[w] = yin ? p.y0[w] : p.rr[w];
+    if (!UNIT && !yin) quot(p.rr, p.d, rd, in, yv);
+#pragma unroll
+    for (int s = 0; s < kMarchC; s++) {
+      if (s < g.c) {
+        float4* im = img + s * g.pts * LP;
+        if (t < g.pts) im[lane] = make_float4(yv[0], yv[1], yv[2], yv[3]);
+        lds_barrier();
+        if (t < g.pts) {
+          const float4 fx = im[t > 0 ? lane - LP : lane], fy = im[t >= g.ex ? lane - g.ex * LP : lane];
+          const float nx[4] = {fx.x, fx.y, fx.z, fx.w}, ny[4] = {fy.x, fy.y, fy.z, fy.w};
+#pragma unroll
+          for (int w = 0; w < 4; w++) {
+            float sum = 0.0f;
+            if (UPPER) {
+              sum = sum + p.v[0] * nx[w];
+              sum = sum + p.v[1] * ny[w];
+              sum = sum + p.v[2] * prev[s][w];
+            } else {
+              sum = sum + p.v[0] * prev[s][w];
+              sum = sum + p.v[1] * ny[w];
+              sum = sum + p.v[2] * nx[w];
+            }
+            prev[s][w] = yv[w];
+            yv[w] = p.rr[w] - sum;
+          }
+          if (!UNIT) quot(yv, p.d, rd, in, yv);
+        }
+      }
+    }
+    if (core && z >= z0) {
+      const unsigned i = (unsigned)(line + plane * (UPPER ? g.nz - 1 - z : z));
+      vstore<float, 4>(yout + (size_t)i * 32 + c0, yv);
+    }
+    // a single sweep's image is written again right after
+    if (g.c == 1) lds_barrier();
+  };
+  for (int z = zs; z < z1; z += 2) {
+    load(b, z + 1);
+    step(a, z);
+    if (z + 1 >= z1) break;
+    load(a, z + 2);
+    step(b, z + 1);
+  }
+}
+
+// Tiles of the xy plane (as few lanes in all as fit kMarchBS points with the
+// halo) and runs of planes (512 workgroups, two a CU, but at least 8 planes).
+static MarchShape march_shape(const TriPlan& P, int c) {
+  MarchShape g;
+  g.n = P.n, g.nx = P.grid[0], g.ny = P.grid[1], g.nz = P.grid[2], g.c = c;
+  long best = -1;
+  g.kx = g.ky = 1;
+  for (int kx = 1; kx <= std::min(g.nx, 64); kx++) {
+    const int ex = ceil_div(g.nx, kx) + c, most = kMarchBS / kMarchLP / ex - c;  // lines of a tile
+    if (most < 1) continue;
+    const int ky = ceil_div(g.ny, most);
+    const long cost = (long)kx * ky * ceil_div((long)kMarchLP * ex * (ceil_div(g.ny, ky) + c), 64);
+    if (best < 0 || cost < best) best = cost, g.kx = kx, g.ky = ky;
+  }
+  g.bx = ceil_div(g.nx, g.kx), g.by = ceil_div(g.ny, g.ky);
+  g.ex = g.bx + c;
+  g.pts = g.ex * (g.by + c);
+  g.mx = ((1u << 20) + g.ex - 1) / g.ex;
+  const int runs = std::max(1, std::min(512 / (kMarchCG * g.kx * g.ky), g.nz / 8));
+  g.bz = ceil_div(g.nz, runs);
+  g.kz = ceil_div(g.nz, g.bz);
+  return g;
+}
+
+static bool jacobi32_march_applies(const TriPlan& P, const float* val) {
+  return P.grid[0] > 0 && P.dia.nd == 3 && P.strict_src == (const void*)val && !(P.stale & TriPlan::kFormDia) &&
+         (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) && P.n <= (1 << 29) && P.grid[0] < 4096 &&
+         P.grid[1] < 4096 && get_option("jacobi_dia", 1) != 0 && get_option("jacobi_pair", 1) != 0;
+}
+
+// yout = c sweeps from yin, or from the first sweep's r / diag where yin is
+// null (yin, r and yout distinct).
+static int jacobi32_march(const TriPlan& P, const float* r, const float* yin, float* yout, int c) {
+  const MarchShape g = march_shape(P, c);
+  const double offd = (double)P.nnz - P.n;
+  TimedRegion tr(P.upper ? "block_jacobi_march_upper" : "block_jacobi_march_lower", c * (64.0 * offd + 32.0 * P.n),
+                 P.dia.bytes(4) + (P.unit_diag ? 0.0 : 4.0 * P.n) + 128.0 * P.n * (yin ? 3.0 : 2.0));
+  const float *dv = P.dia.val.as<float>(), *dg = P.dval.as<float>();
+  const int nb = kMarchCG * g.kx * g.ky * g.kz, bs = ceil_div(g.pts * kMarchLP, 64) * 64;
+  const size_t lds = sizeof(float4) * g.pts * kMarchLP * c;
+#define LACE_MARCH(UP, UN) jacobi32_march_kernel<UP, UN><<<nb, bs, lds, stream()>>>(g, dv, dg, r, yin, yout)
+  if (P.upper) {
+    if (P.unit_diag) LACE_MARCH(true, true);
+    else LACE_MARCH(true, false);
+  } else {
+    if (P.unit_diag) LACE_MARCH(false, true);
+    else LACE_MARCH(false, false);
+  }
+#undef LACE_MARCH
+  LACE_HIP(hipGetLastError());
+  return DEV_SUCCESS;
+}
+
 template <typename T>
 static int jacobi32_sweep(const TriPlan& P, const T* val, const T* r, const T* yin, T* yout) {
   const int nb = ceil_div(P.n, Lanes<T>::RPB);
@@ -691,6 +871,19 @@ static int jacobi32_solve(const TriPlan& P, const T* val, const T* r, T* y, T* t
   // of L writes y when L - 1 - idx is even, tmp otherwise, so the last
   // lands in y and no launch reads its own output.
   const int K = sweeps - 1;
+  if constexpr (sizeof(T) == 4) {
+    if (K >= 1 && r != y && r != tmp && jacobi32_march_applies(P, val)) {
+      // launches of equal length, ping-ponging so that the last lands in y
+      const int L = ceil_div(K, kMarchC);
+      const T* src = nullptr;
+      for (int l = 0; l < L; l++) {
+        T* o = (L - 1 - l) % 2 == 0 ? y : tmp;
+        LACE_TRY(jacobi32_march(P, r, src, o, K * (l + 1) / L - K * l / L));
+        src = o;
+      }
+      return DEV_SUCCESS;
+    }
+  }
   const bool pair = jacobi32_pair_applies<T>(P, val);
   const int L = pair ? (K + 1) / 2 : K;
   auto out_of = [&](int idx) { return ((L - 1 - idx) % 2 == 0) ? y : tmp; };

@@ -211,14 +211,6 @@ int TriPlan::copy_ring(const TriPlan& o) {
 
 namespace {
 
-// Workgroup barrier that orders LDS only: global loads issued ahead stay in
-// flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // A chunk's data in flight: lane t holds row t's entries.
 template <typename T, int NG>
 struct RingStage {

@@ -1,0 +1,74 @@
+"""32-column Jacobi sweeps, several to a launch plane by plane (option
+"jacobi_pair" 1): bit-identical to one sweep per launch (0) and to the
+single-vector solve.  Grids narrower than the sweeps' reach, of one and several
+tiles along each axis, of one and several runs of planes with a short last one;
+one launch and several; both factors and directions; infinities and NaN; a
+pattern with gaps, which keeps the other kernels."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(2, 2, 2), (4, 3, 5), (9, 3, 17), (30, 30, 9), (31, 33, 8), (61, 18, 40), (17, 70, 25), (200, 5, 19), (3, 3, 100)]
+
+
+def _both(gpu, P, R, sweeps, trans):
+    out = []
+    for on in (1, 0):
+        gpu.check(gpu.lib().lace_set_option(b"jacobi_pair", on))
+        try:
+            out.append(P.apply_block(R, gpu.TRSV_JACOBI, sweeps=sweeps, trans=trans))
+        finally:
+            gpu.check(gpu.lib().lace_set_option(b"jacobi_pair", 1))
+    return out
+
+
+@pytest.mark.parametrize("dims", GRIDS)
+def test_march_matches_single_sweeps(gpu, orc, dims):
+    A = orc.convdiff3d(*dims)
+    rng = np.random.default_rng(7)
+    A = orc.CSR(A.n_rows, A.n_cols, A.row, A.col, A.val * rng.uniform(0.75, 1.25, A.nnz))
+    print(f"march: {dims}", flush=True)
+    P = gpu.ParILU(gpu.HostCSR.from_csr(A), gpu.LACE_F32)
+    P.sweeps(3)
+    R = rng.standard_normal((A.n_rows, 32)).astype(np.float32)
+    for trans in (0, 1):
+        for k in (1, 2, 3, 4, 5, 6, 9, 10):
+            a, b = _both(gpu, P, R, k, trans)
+            assert np.array_equal(a, b), (trans, k)
+        z = P.apply(R[:, 13].copy(), gpu.TRSV_JACOBI, sweeps=5, trans=trans)
+        assert np.array_equal(_both(gpu, P, R, 5, trans)[0][:, 13], z)
+
+
+def test_march_special_values_and_gaps(gpu, orc):
+    A = orc.convdiff3d(24, 19, 21)
+    rng = np.random.default_rng(3)
+    ri = A.rowidx()
+    keep = (ri == A.col) | (rng.random(A.nnz) >= 0.1)
+    row = np.zeros(A.n_rows + 1, dtype=np.int32)
+    np.add.at(row, ri[keep] + 1, 1)
+    gaps = orc.CSR(A.n_rows, A.n_cols, np.cumsum(row).astype(np.int32), A.col[keep].copy(), A.val[keep].copy())
+    R = rng.standard_normal((A.n_rows, 32)).astype(np.float32)
+    R[5, 3], R[4000, 17], R[9000, 31], R[70, 0] = np.inf, np.nan, -np.inf, -0.0
+    for M in (A, gaps):
+        P = gpu.ParILU(gpu.HostCSR.from_csr(M), gpu.LACE_F32)
+        P.sweeps(3)
+        for trans in (0, 1):
+            a, b = _both(gpu, P, R, 5, trans)
+            assert np.array_equal(a, b, equal_nan=True), trans
+
+
+def test_march_quotients(gpu, orc):
+    """Right-hand sides from the subnormal range to the largest: the sweeps'
+    quotients round as IEEE division does, which the one-sweep launches use."""
+    A = orc.convdiff3d(16, 8, 12)
+    rng = np.random.default_rng(9)
+    P = gpu.ParILU(gpu.HostCSR.from_csr(A), gpu.LACE_F32)
+    P.sweeps(3)
+    R = rng.standard_normal((A.n_rows, 32)) * 2.0 ** rng.integers(-150, 120, (A.n_rows, 32))
+    R = R.astype(np.float32)
+    for k in (2, 5):
+        a, b = _both(gpu, P, R, k, 0)
+        assert np.array_equal(a, b, equal_nan=True), k
+        z = P.apply(R[:, 4].copy(), gpu.TRSV_JACOBI, sweeps=k)
+        assert np.array_equal(a[:, 4], z, equal_nan=True), k
