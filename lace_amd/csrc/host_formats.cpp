@@ -825,13 +825,19 @@ int data_zfrobenius(data_d_matrix A, dataType* res) {
 }
 
 // Sparse x sparse product C = alpha*A*B with sorted rows (the reference
-// wraps mkl_sparse_spmm, blas/zspmm.cpp:47-167).  Dense-marker row merge.
+// wraps mkl_sparse_spmm, blas/zspmm.cpp:47-167).
 int data_z_spmm(dataType alpha, data_d_matrix A, data_d_matrix B, data_d_matrix* C) {
   const int m = A.num_rows, n = B.num_cols;
   std::vector<int> crow(m + 1, 0), ccol;
   std::vector<double> cval;
-  ccol.reserve((size_t)3 * (A.row[m] + (size_t)m));
-  cval.reserve((size_t)3 * (A.row[m] + (size_t)m));
+  if (m > 0) {
+    // room for three times A and a row more, and for no more than the products
+    size_t products = 0;
+    for (int p = 0; p < A.row[m]; p++) products += B.row[A.col[p] + 1] - B.row[A.col[p]];
+    const size_t room = std::min(products, (size_t)3 * ((size_t)A.row[m] + m));
+    ccol.reserve(room);
+    cval.reserve(room);
+  }
   product_rows(A, B, [&](int i, int cnt, const int* list, const double* acc) {
     for (int a = 0; a < cnt; a++) {
       ccol.push_back(list[a]);

@@ -156,6 +156,17 @@ def test_ilures_and_spgemm_match_oracle(lace, orc):
     assert np.allclose(cv, ref.val, rtol=1e-15, atol=1e-15)
 
 
+def test_product_of_empty_matrices(lace):
+    """A matrix without rows may have null arrays; the product then has no
+    rows either, whatever the other factor is."""
+    E, Cm = lace.DMatrix(), lace.DMatrix()
+    E.storage_type = lace.Magma_CSR
+    for B in (lace.DMatrix(), lace.HostCSR([0, 1], [0], [2.0]).m):
+        lace.check(lace.lib().data_z_spmm(1.0, E, B, C.byref(Cm)))
+        assert Cm.num_rows == 0 and Cm.num_cols == B.num_cols and Cm.nnz == 0 and Cm.row[0] == 0
+        lace.lib().data_zmfree(C.byref(Cm))
+
+
 def test_exact_ilu0_matches_oracle(lace, orc):
     A = orc.convdiff3d(6, 6, 5)
     H = lace.HostCSR.from_csr(A)
