@@ -1435,16 +1435,13 @@ int data_zilures(data_d_matrix A, data_d_matrix L, data_d_matrix U, data_d_matri
   LACE_TRY(rc);
   double r = 0.0, nl = 0.0;
   for (int i = 0; i < n; i++) {
-    int lo = LU->row[i];
-    for (int k = A.row[i]; k < A.row[i + 1]; k++) {
-      // LU rows are sorted: on from the previous column's place, or from the
-      // row's start where A's columns are not in order
-      const int c = A.col[k];
-      if (k > A.row[i] && c < A.col[k - 1]) lo = LU->row[i];
-      while (lo < LU->row[i + 1] && LU->col[lo] < c) lo++;
-      if (lo < LU->row[i + 1] && LU->col[lo] == c) {
-        double t = LU->val[lo] - A.val[k];
-        LU->val[lo] = t;
+    const int l0 = LU->row[i], a0 = A.row[i];
+    RowPlaces places(LU->col + l0, LU->row[i + 1] - l0);
+    for (int k = a0; k < A.row[i + 1]; k++) {
+      const int q = places.next(A.col[k]);
+      if (q >= 0) {
+        double t = LU->val[l0 + q] - A.val[k];
+        LU->val[l0 + q] = t;
         nl += t * t;
       }
     }
@@ -1471,14 +1468,12 @@ int lu_residual(const data_d_matrix& A, const data_d_matrix& L, const data_d_mat
   std::vector<double> row(Ur.num_cols);
   product_rows(L, Ur, [&](int i, int cnt, const int* list, const double* acc) {
     for (int a = 0; a < cnt; a++) row[a] = acc[list[a]];
-    int at = 0;
+    RowPlaces places(list, cnt);
     for (int k = A.row[i]; k < A.row[i + 1]; k++) {
-      const int c = A.col[k];
-      if (k > A.row[i] && c < A.col[k - 1]) at = 0;
-      while (at < cnt && list[at] < c) at++;
-      if (at < cnt && list[at] == c) {
-        const double t = row[at] - A.val[k];
-        row[at] = t;
+      const int q = places.next(A.col[k]);
+      if (q >= 0) {
+        const double t = row[q] - A.val[k];
+        row[q] = t;
         nl += t * t;
       }
     }

@@ -167,6 +167,66 @@ def test_product_of_empty_matrices(lace):
         lace.lib().data_zmfree(C.byref(Cm))
 
 
+def _rows(orc, n, lists, seed=0):
+    """CSR matrix with the given column lists, in their order."""
+    row = np.concatenate([[0], np.cumsum([len(c) for c in lists])]).astype(np.int32)
+    col = np.concatenate(lists).astype(np.int32)
+    return orc.CSR(n, n, row, col, np.random.default_rng(seed).uniform(0.5, 1.5, len(col)))
+
+
+@pytest.mark.parametrize("kind", ["wide", "edge", "narrow", "dense", "many", "repeated"])
+def test_product_rows_of_every_kind(lace, orc, kind):
+    """Rows of a product whose columns lie far apart, just as far as the bits
+    are passed over and one less, of 127 to 129 products, and dense ones, each
+    after the other kinds have used the same work arrays."""
+    n = {"wide": 600000, "edge": 262146, "narrow": 262146}.get(kind, 300)
+    i = np.arange(n)
+    if kind in ("wide", "edge", "narrow"):
+        far = {"wide": n - 1, "edge": 262144, "narrow": 262143}[kind]
+        lists = [np.array([k]) for k in i]
+        for k in (0, 5, 70000):
+            lists[k] = np.unique([0, 1, k, 63, 64, 4095, 4096, far])
+    elif kind == "dense":
+        lists = [i] * n
+    elif kind == "many":
+        lists = [np.unique([k] + list(range(0, 11 + k % 3))) for k in i]
+    else:
+        lists = [np.array([k, 0, 0, k, 7]) for k in i]
+    A, B = _rows(orc, n, lists, 1), _rows(orc, n, lists, 2)
+    Cm = lace.DMatrix()
+    Ah, Bh = lace.HostCSR.from_csr(A), lace.HostCSR.from_csr(B)
+    lace.check(lace.lib().data_z_spmm(-1.5, Ah.m, Bh.m, C.byref(Cm)))
+    cr, cc, cv = lace.owned_to_numpy(Cm)
+    ref = orc.spgemm(A, B)
+    assert np.array_equal(cr, ref.row) and np.array_equal(cc, ref.col)
+    # sums of the same products in the same order, then scaled
+    assert np.allclose(cv, -1.5 * ref.val, rtol=1e-14, atol=0)
+
+
+@pytest.mark.parametrize("order", ["ascending", "descending", "shuffled"])
+def test_ilures_takes_columns_in_any_order(lace, orc, order):
+    """The norms do not depend on the order of A's columns (but for the
+    rounding of their sums); rows as long as the matrix among them."""
+    n = 240
+    rng = np.random.default_rng(4)
+    lists = [np.arange(n) if k % 3 == 0 else np.unique(np.append(rng.integers(0, n, 5), k)) for k in range(n)]
+    A = _rows(orc, n, lists, 3)
+    Lf, Uf = orc.csr_split(A, False, orc.DIAG_UNIT), orc.csr_split(A, True, orc.DIAG_VALUE)
+    want, nlwant = orc.ilures(A, Lf, Uf)
+    col, val = A.col.copy(), A.val.copy()
+    for k in range(n):
+        s = slice(A.row[k], A.row[k + 1])
+        p = {"ascending": np.arange, "descending": lambda m: np.arange(m)[::-1], "shuffled": rng.permutation}[order](s.stop - s.start)
+        col[s], val[s] = col[s][p], val[s][p]
+    Ah = lace.HostCSR(A.row, col, val)
+    Lh, Uh = lace.HostCSR.from_csr(Lf), lace.HostCSR.from_csr(Uf)
+    Lh.m.storage_type, Uh.m.storage_type = lace.Magma_CSRL, lace.Magma_CSRU
+    LU, r, nl = lace.DMatrix(), C.c_double(), C.c_double()
+    lace.check(lace.lib().data_zilures(Ah.m, Lh.m, Uh.m, C.byref(LU), C.byref(r), C.byref(nl)))
+    lace.owned_to_numpy(LU)
+    assert abs(r.value - want) <= 1e-12 * want and abs(nl.value - nlwant) <= 1e-12 * nlwant
+
+
 def test_exact_ilu0_matches_oracle(lace, orc):
     A = orc.convdiff3d(6, 6, 5)
     H = lace.HostCSR.from_csr(A)
