@@ -56,6 +56,9 @@ int num_cus();
 // Device address of the allocation-free entry point's scratch array on
 // this GPU, looked up once per device (noalloc.hip).
 int noalloc_setup(int device);
+// LDS sizes of the one-workgroup exact solves on the present device
+// (trsv_ring.hip).
+int ring_setup();
 // Kernel-shape option set through lace_set_option (dflt when unset).
 int get_option(const char* name, int dflt);
 

@@ -54,6 +54,7 @@ static int init_device(int dev) {
   g_cus = prop.multiProcessorCount;
   // this GPU's allocation-free scratch address (noalloc.hip)
   LACE_TRY(noalloc_setup(dev));
+  LACE_TRY(ring_setup());
   return DEV_SUCCESS;
 }
 

@@ -368,16 +368,36 @@ bool ring_ready(const TriPlan& P) {
          get_option("trsv_exact_rows", 512) == 512;
 }
 
+// The kernels' LDS is past what a launch may ask for by itself: allowed for
+// each of them, on the present device, when the library is initialised on it.
+template <typename T, int NG, int W, bool DIRECT>
+static int ring_allow() {
+  LACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(tri_ring_kernel<T, NG, W, DIRECT>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               kRingBytes + 16 + (int)sizeof(uint2) * kRingDescs));
+  return DEV_SUCCESS;
+}
+template <typename T, int W, bool DIRECT>
+static int ring_allow_groups() {
+  LACE_TRY((ring_allow<T, 1, W, DIRECT>()));
+  LACE_TRY((ring_allow<T, 2, W, DIRECT>()));
+  return ring_allow<T, 4, W, DIRECT>();
+}
+template <typename T>
+static int ring_allow_all() {
+  LACE_TRY((ring_allow_groups<T, 8, false>()));
+  LACE_TRY((ring_allow_groups<T, 8, true>()));
+  LACE_TRY((ring_allow_groups<T, 16, false>()));
+  return ring_allow_groups<T, 16, true>();
+}
+int ring_setup() {
+  LACE_TRY(ring_allow_all<float>());
+  return ring_allow_all<double>();
+}
+
 template <typename T, int NG, int W, bool DIRECT>
 static int ring_launch(const TriPlan& P, const T* rhs, T* out) {
   const size_t lds = kRingBytes + 16 + sizeof(uint2) * P.rchunks;
-  static bool set = false;
-  if (!set) {
-    LACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(tri_ring_kernel<T, NG, W, DIRECT>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 kRingBytes + 16 + (int)sizeof(uint2) * kRingDescs));
-    set = true;
-  }
   tri_ring_kernel<T, NG, W, DIRECT><<<1, W * 64, lds, stream()>>>(
       P.nlev, P.rchunks, reinterpret_cast<const uint2*>(P.rdesc()), P.rval.as<T>(), reinterpret_cast<const ushort4*>(P.ridx()), rhs, P.rdiag.as<T>(),
       P.rperm(), out);
