@@ -683,8 +683,12 @@ int lace_block_panel_qr(int n, int r0, const double *W, double *Y, double *Tb, d
  * are still in the L2 cache (0: natural row order).  "jacobi_pair" (0 or 1,
  * default 1): the 32-right-hand-side Jacobi sweeps on the diagonal form run
  * two to a launch, each row forming the first sweep's result at the rows
- * it reads (0: one sweep per launch).  Every choice gives bit-identical
- * results.  "matlab_log" (0 or 1, default 1): the
+ * it reads, or more to a launch as "jacobi_march" says (0: one sweep per
+ * launch).  "jacobi_march" (0..2, default 1): the FP32 sweeps of full 7-point
+ * factors run up to four coupled ones to a launch, plane by plane of the
+ * grid, where that is expected to be faster (grids of more than about 130000
+ * points and three sweeps or more; 0: never, 2: wherever the form exists).
+ * Every choice gives bit-identical results.  "matlab_log" (0 or 1, default 1): the
  * drop-in FGMRES entry points print the reference's MATLAB-syntax progress
  * lines to stdout (src/fgmres.cpp:71,178,430; src/fgmres_householder_restart.cpp:
  * 70,81,196,231,707) -- "FGMRES_Householders_partrsv_search(j) = |g_j|;" etc.,

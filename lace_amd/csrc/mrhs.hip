@@ -738,10 +738,46 @@ static MarchShape march_shape(const TriPlan& P, int c) {
   return g;
 }
 
-static bool jacobi32_march_applies(const TriPlan& P, const float* val) {
-  return P.grid[0] > 0 && P.dia.nd == 3 && P.strict_src == (const void*)val && !(P.stale & TriPlan::kFormDia) &&
-         (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) && P.n <= (1 << 29) && P.grid[0] < 4096 &&
-         P.grid[1] < 4096 && get_option("jacobi_dia", 1) != 0 && get_option("jacobi_pair", 1) != 0;
+// Whether that is ahead of pairs of sweeps, by the points it forms (halo and
+// early planes included, two to one for four sweeps on a cube) and by its
+// workgroups: launches that fill the chip once or twice over, since one that
+// fills half of a round more takes the time of the whole round.  Five, four and
+// three sweeps (c = 4, 3, 2; six: 2 and 3) of L and U, pairs -> march:
+//   12^3 (4 workgroups) 27 -> 48 us, 32^3 (64) 95 -> 119, 56^3 (336) 148 -> 166,
+//   (252, c = 3) 135 -> 117, 200 x 200 x 4 (480) 142 -> 115, six 164 -> 155;
+//   64^3, c = 2: 123 -> 141; six: 200 -> 242;
+//   72 x 72 x 64 480 -> 476, c = 3 457 -> 436, six 514 -> 526, 80 x 72 x 64
+//   510 -> 445, c = 2 442 -> 388, six 544 -> 504 (past 2^18 rows the four
+//   vectors no longer stay in the last cache, and what counts is what is moved);
+//   128^3 1765 -> 1440;
+//   5 x 5 x 20000, whose tile is 81 points: 583 -> 731.
+// A single sweep has nothing to save (64^3 106 -> 117 us, 100^3 790 -> 808).
+static bool march_pays(const MarchShape& g) {
+  const double formed = (double)g.pts * g.kx * g.ky * (g.nz + (g.kz - 1.0) * g.c) / g.n;
+  if (g.n > (1 << 18)) return g.c >= (g.n < 350000 ? 3 : 2) && g.pts >= 128 && formed <= 2.5;
+  const int wgs = kMarchCG * g.kx * g.ky * g.kz;
+  const double most = g.c == 1 ? 0.0 : g.c == 2 ? 1.3 : g.n < (1 << 17) ? 1.6 : 2.2;
+  return formed <= most && ((wgs >= 192 && wgs <= 256) || wgs >= (g.c == 2 ? 400 : 440));
+}
+
+// Launches of K coupled sweeps, of equal length but for one: launch l's sweeps.
+static int march_launches(int K) { return ceil_div(K, kMarchC); }
+static int march_sweeps(int K, int l) {
+  const int L = march_launches(K);
+  return K * (l + 1) / L - K * l / L;
+}
+
+// Option "jacobi_march": 1 where it pays for every launch of the K sweeps, 2
+// wherever there is such a form, 0 never.
+static bool jacobi32_march_applies(const TriPlan& P, const float* val, int K) {
+  const int march = get_option("jacobi_march", 1);
+  const bool there = K >= 1 && P.grid[0] > 0 && P.dia.nd == 3 && P.strict_src == (const void*)val &&
+                     !(P.stale & TriPlan::kFormDia) && (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) &&
+                     P.n <= (1 << 29) && P.grid[0] < 4096 && P.grid[1] < 4096 && get_option("jacobi_dia", 1) != 0 &&
+                     get_option("jacobi_pair", 1) != 0;
+  if (!there || march != 1) return there && march == 2;
+  const int shortest = K / march_launches(K), longest = ceil_div(K, march_launches(K));
+  return march_pays(march_shape(P, longest)) && (shortest == longest || march_pays(march_shape(P, shortest)));
 }
 
 // yout = c sweeps from yin, or from the first sweep's r / diag where yin is
@@ -872,13 +908,13 @@ static int jacobi32_solve(const TriPlan& P, const T* val, const T* r, T* y, T* t
   // lands in y and no launch reads its own output.
   const int K = sweeps - 1;
   if constexpr (sizeof(T) == 4) {
-    if (K >= 1 && r != y && r != tmp && jacobi32_march_applies(P, val)) {
-      // launches of equal length, ping-ponging so that the last lands in y
-      const int L = ceil_div(K, kMarchC);
+    if (r != y && r != tmp && jacobi32_march_applies(P, val, K)) {
+      // ping-ponging so that the last lands in y
+      const int L = march_launches(K);
       const T* src = nullptr;
       for (int l = 0; l < L; l++) {
         T* o = (L - 1 - l) % 2 == 0 ? y : tmp;
-        LACE_TRY(jacobi32_march(P, r, src, o, K * (l + 1) / L - K * l / L));
+        LACE_TRY(jacobi32_march(P, r, src, o, march_sweeps(K, l)));
         src = o;
       }
       return DEV_SUCCESS;

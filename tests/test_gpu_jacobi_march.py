@@ -1,9 +1,11 @@
 """32-column Jacobi sweeps, several to a launch plane by plane (option
-"jacobi_pair" 1): bit-identical to one sweep per launch (0) and to the
-single-vector solve.  Grids narrower than the sweeps' reach, of one and several
+"jacobi_march" 2: wherever there is such a form): bit-identical to one sweep
+per launch ("jacobi_pair" 0) and to the single-vector solve.  Grids narrower than the sweeps' reach, of one and several
 tiles along each axis, of one and several runs of planes with a short last one;
 one launch and several; both factors and directions; infinities and NaN; a
 pattern with gaps, which keeps the other kernels."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -12,15 +14,56 @@ pytestmark = pytest.mark.gpu
 GRIDS = [(2, 2, 2), (4, 3, 5), (9, 3, 17), (30, 30, 9), (31, 33, 8), (61, 18, 40), (17, 70, 25), (200, 5, 19), (3, 3, 100)]
 
 
+def _opt(gpu, name, value):
+    gpu.check(gpu.lib().lace_set_option(name, value))
+
+
 def _both(gpu, P, R, sweeps, trans):
     out = []
-    for on in (1, 0):
-        gpu.check(gpu.lib().lace_set_option(b"jacobi_pair", on))
+    for march, pair in ((2, 1), (1, 0)):
+        _opt(gpu, b"jacobi_march", march)
+        _opt(gpu, b"jacobi_pair", pair)
         try:
             out.append(P.apply_block(R, gpu.TRSV_JACOBI, sweeps=sweeps, trans=trans))
         finally:
-            gpu.check(gpu.lib().lace_set_option(b"jacobi_pair", 1))
+            _opt(gpu, b"jacobi_march", 1)
+            _opt(gpu, b"jacobi_pair", 1)
     return out
+
+
+def _launches(gpu, P, R, sweeps):
+    """Launches of L's sweeps by kind: plane by plane, pairs, single ones."""
+    lib = gpu.lib()
+    gpu.check(lib.lace_timing_enable(1))
+    gpu.check(lib.lace_timing_reset())
+    try:
+        P.apply_block(R, gpu.TRSV_JACOBI, sweeps=sweeps)
+        out = []
+        for kind in (b"march", b"pair", b"sweep"):
+            calls = C.c_long(0)
+            lib.lace_timing_get_calls(b"block_jacobi_" + kind + b"_lower", C.byref(calls))
+            out.append(calls.value)
+    finally:
+        gpu.check(lib.lace_timing_enable(0))
+    return tuple(out)
+
+
+@pytest.mark.parametrize("dims,sweeps,want", [
+    # few workgroups: the pair kernels
+    ((2, 2, 2), 5, (0, 0, 4)),  # (no diagonal form)
+    ((16, 16, 16), 5, (0, 2, 0)), ((16, 16, 16), 4, (0, 1, 1)), ((10, 10, 40), 3, (0, 1, 0)),
+    ((5, 5, 4000), 5, (0, 2, 0)), ((64, 64, 16), 5, (0, 2, 0)), ((56, 56, 56), 5, (0, 2, 0)),
+    # a single coupled sweep has nothing to save
+    ((72, 72, 72), 2, (0, 0, 1)),
+    # the chip is full
+    ((200, 200, 4), 5, (1, 0, 0)), ((200, 200, 4), 6, (2, 0, 0)), ((72, 72, 72), 5, (1, 0, 0)), ((72, 72, 72), 3, (1, 0, 0)),
+    ((72, 72, 72), 6, (2, 0, 0))])
+def test_march_only_where_it_pays(gpu, orc, dims, sweeps, want):
+    A = orc.convdiff3d(*dims)
+    P = gpu.ParILU(gpu.HostCSR.from_csr(A), gpu.LACE_F32)
+    P.sweeps(2)
+    R = np.random.default_rng(1).standard_normal((A.n_rows, 32)).astype(np.float32)
+    assert _launches(gpu, P, R, sweeps) == want
 
 
 @pytest.mark.parametrize("dims", GRIDS)
