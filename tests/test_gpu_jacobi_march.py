@@ -115,3 +115,21 @@ def test_march_quotients(gpu, orc):
         assert np.array_equal(a, b, equal_nan=True), k
         z = P.apply(R[:, 4].copy(), gpu.TRSV_JACOBI, sweeps=k)
         assert np.array_equal(a[:, 4], z, equal_nan=True), k
+
+
+def test_march_zeros(gpu, orc):
+    """Zeros of either sign, alone and beside quotients below the normal range:
+    the same bits as one sweep per launch."""
+    A = orc.convdiff3d(16, 8, 12)
+    rng = np.random.default_rng(11)
+    P = gpu.ParILU(gpu.HostCSR.from_csr(A), gpu.LACE_F32)
+    P.sweeps(3)
+    R = rng.standard_normal((A.n_rows, 32)).astype(np.float32)
+    R[rng.random(R.shape) < 0.6] = 0.0
+    R[rng.random(R.shape) < 0.2] = -0.0
+    R[: A.n_rows // 2] = -0.0
+    R[rng.random(R.shape) < 0.05] = np.float32(3e-39)
+    for k in (2, 3, 5):
+        for trans in (0, 1):
+            a, b = _both(gpu, P, R, k, trans)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (k, trans)
