@@ -666,11 +666,13 @@ int lace_block_panel_qr(int n, int r0, const double *W, double *Y, double *Tb, d
  * the last sweep of L (diagonal form only).  "jacobi_dia_vec" (0 or 1,
  * default 1): Jacobi sweeps on the diagonal form take a 16-byte word of
  * rows per thread (4 FP32, 2 FP64) where n is a multiple of a word and the
- * vectors are 16-byte aligned, and two or more sweeps of a factor whose rows
- * are the points of a grid with an entry for every neighbour one step back
- * along each axis (the factors of 5- and 7-point stencils) run up to five to
- * a launch, a workgroup per box of the grid (0: one row per thread, one
- * sweep per launch).  "jacobi_pipe" (0 or
+ * vectors are 16-byte aligned (0: one row per thread, one sweep per launch).
+ * "jacobi_tile" (0..2, default 1; with "jacobi_dia_vec"): two or more sweeps
+ * of a factor whose rows are the points of a grid with an entry for every
+ * neighbour one step back along each axis (the factors of 5- and 7-point
+ * stencils) run up to five to a launch, a workgroup per box of the grid,
+ * where that is expected to be faster (0: never, 2: wherever the form
+ * exists).  "jacobi_pipe" (0 or
  * 1, default 0): a ParILU apply with k >= 3 Jacobi sweeps, both factors on
  * the diagonal form, runs sweeps 2..k of each factor in one launch (tiles
  * in ticket order, each waiting on the tiles it reads through progress

@@ -360,7 +360,7 @@ extern "C" int lace_set_option(const char* name, int value) {
     LACE_REQUIRE(value == 0 || value == 1, DEV_ERR_ILLEGAL_VALUE, "%s must be 0 or 1 (have %d)", name, value);
   } else if (key == "trsv_exact_wgs_per_cu") {
     LACE_REQUIRE(value >= 0 && value <= 16, DEV_ERR_ILLEGAL_VALUE, "%s must be 0..16 (have %d)", name, value);
-  } else if (key == "trsv_exact_ring" || key == "jacobi_march") {
+  } else if (key == "trsv_exact_ring" || key == "jacobi_march" || key == "jacobi_tile") {
     LACE_REQUIRE(value >= 0 && value <= 2, DEV_ERR_ILLEGAL_VALUE, "%s must be 0..2 (have %d)", name, value);
   } else if (key == "trsv_exact") {
     LACE_REQUIRE(value == 0 || value == 1, DEV_ERR_ILLEGAL_VALUE, "%s must be 0 or 1 (have %d)", name, value);

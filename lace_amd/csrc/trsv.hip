@@ -1844,9 +1844,9 @@ int ParILU::prepare(lace_trsv_kind_t kind, int trans, bool block, int sweeps) {
     TriPlan& a = trans ? lowerT : lower;
     TriPlan& b = trans ? upperT : upper;
     // sweeps on boxes that read the 16-bit words need no FP32 copies
-    const bool words = !block && sweeps >= 2 && get_option("jacobi_pipe", 0) == 0;
-    if (!(words && jacobi_tile16(a))) LACE_TRY(a.ensure_forms(jacobi_forms(a, block)));
-    if (!(words && jacobi_tile16(b))) LACE_TRY(b.ensure_forms(jacobi_forms(b, block)));
+    const bool words = !block && get_option("jacobi_pipe", 0) == 0;
+    if (!(words && jacobi_tile16(a, sweeps))) LACE_TRY(a.ensure_forms(jacobi_forms(a, block)));
+    if (!(words && jacobi_tile16(b, sweeps))) LACE_TRY(b.ensure_forms(jacobi_forms(b, block)));
   }
   return DEV_SUCCESS;
 }

@@ -248,18 +248,39 @@ static void tile_dispatch(const TriPlan& P, const TS* dia, const TS* dval, const
 #undef LACE_TILE_CASE
 }
 
-bool jacobi_tile16(const TriPlan& P) {
+static bool has16(const TriPlan& P) {
   return P.grid[0] > 0 && P.dia16_fmt != LACE_F32 && P.dia16_src != nullptr && P.dia16_src == P.strict_src &&
          P.upper != P.unit_diag && (double)P.n * sizeof(float) < 2147483648.0 &&
          get_option("jacobi_dia16", 1) != 0 && get_option("jacobi_dia", 1) != 0 &&
          get_option("jacobi_dia_vec", 1) != 0;
 }
 
+// Option "jacobi_tile": 1 where boxes are ahead of one-sweep launches, 2
+// wherever there is such a form, 0 never.  They are ahead at two sweeps and
+// more but on large 3-D grids whose lines do not keep the 16-byte word of four
+// rows: there a unit is one row, whose loads, 2 bytes wide for 16-bit words,
+// cost more than one coupled sweep saves, and in 16 bits more than two save;
+// below these sizes the launches saved make up for it.  Two sweeps of L and U,
+// one-sweep launches -> boxes: 77 x 53 x 100 FP32 9.4 -> 12.3 us, 61 x 60 x 61
+// 12.4 -> 10.7, 127 x 129 x 128 FP32 24 -> 29, BF16 22 -> 35, FP64 41 -> 36;
+// three: 127 x 129 x 128 BF16 32.7 -> 40.6, FP32 39 -> 35, 90^3 BF16 18.7 ->
+// 15.8; four, BF16 there 55 -> 51.
+static bool tile_pays(const TriPlan& P, int W, int sweeps, bool d16) {
+  const int tile = get_option("jacobi_tile", 1);
+  if (sweeps < 2 || tile != 1) return sweeps >= 2 && tile == 2;
+  if (P.dia.nd != 3 || W != 4 || P.grid[0] % 4 == 0) return true;
+  return sweeps == 2 ? P.n < (1 << 18) : sweeps > 3 || !d16 || P.n < (1 << 20);
+}
+
+bool jacobi_tile16(const TriPlan& P, int sweeps) { return has16(P) && tile_pays(P, 4, sweeps, true); }
+
 template <typename T>
 bool jacobi_tile_ready(const TriPlan& P, const T* val, int sweeps) {
-  if (sweeps < 2 || P.strict_src != (const void*)val) return false;
-  if (sizeof(T) == 4 && jacobi_tile16(P)) return true;
-  return P.grid[0] > 0 && !(P.stale & TriPlan::kFormDia) && (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) &&
+  if (P.grid[0] == 0 || P.strict_src != (const void*)val) return false;
+  const bool d16 = sizeof(T) == 4 && has16(P);
+  if (!tile_pays(P, 16 / (int)sizeof(T), sweeps, d16)) return false;
+  if (d16) return true;
+  return !(P.stale & TriPlan::kFormDia) && (P.unit_diag || !(P.stale & TriPlan::kFormDiag)) &&
          (double)P.n * sizeof(T) < 2147483648.0 && get_option("jacobi_dia", 1) != 0 &&
          get_option("jacobi_dia_vec", 1) != 0;
 }
@@ -269,7 +290,7 @@ int jacobi_tile(const TriPlan& P, const T* r, const T* yin, T* yout, int c) {
   constexpr int W = 16 / (int)sizeof(T);
   const auto al16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
   const bool vec = P.grid[0] % W == 0 && al16(r) && al16(yin) && al16(yout);
-  const bool d16 = sizeof(T) == 4 && jacobi_tile16(P);
+  const bool d16 = sizeof(T) == 4 && has16(P);
   const double es = sizeof(T), n = P.n, fs = d16 ? 2.0 : es;
   TimedRegion tr(P.upper ? "trsv_jacobi_sweep_upper" : "trsv_jacobi_sweep_lower", 0.0,
                  (P.dia.nd + (P.unit_diag ? 0 : 1)) * fs * n + (d16 ? n : 0.0) + (yin ? 3.0 : 2.0) * es * n, true);

@@ -21,13 +21,14 @@ struct TileShape {
   unsigned mx, my;    // 2^20 / nux and 2^20 / ey, rounded up
 };
 
-// Whether the sweeps on boxes of P read the 16-bit diagonal form (and no
-// FP32 copy of it).
-bool jacobi_tile16(const TriPlan& P);
+// Whether `sweeps` Jacobi sweeps of P run on boxes that read the 16-bit
+// diagonal form (and no FP32 copy of it).
+bool jacobi_tile16(const TriPlan& P, int sweeps);
 
-// Whether `sweeps` Jacobi sweeps of P with the value array val can run on
-// boxes: a grid with every neighbour present (TriPlan::grid), its diagonal
-// form current, and byte offsets of a vector within 31 bits.
+// Whether `sweeps` Jacobi sweeps of P with the value array val run on boxes:
+// a grid with every neighbour present (TriPlan::grid), its diagonal form
+// current, byte offsets of a vector within 31 bits, and ahead of one-sweep
+// launches there.
 template <typename T>
 bool jacobi_tile_ready(const TriPlan& P, const T* val, int sweeps);
 

@@ -1,6 +1,7 @@
 """Several Jacobi sweeps per launch on boxes of the grid (option
-"jacobi_dia_vec" 1): bit-identical to one-sweep launches of a row per thread
-(0), which the other tests tie to the oracle.  Grids whose sides fall short of, meet and pass the boxes'
+"jacobi_tile" 2: wherever there is such a form): bit-identical to one-sweep
+launches of a row per thread ("jacobi_dia_vec" 0), which the other tests tie
+to the oracle.  Grids whose sides fall short of, meet and pass the boxes'
 (16 x 8 x 8, 12 x 12 x 12, 64 x 24, ...), lines that do and do not keep the
 16-byte word, every factor storage, transposed solves, one launch and
 several, a pattern with gaps (which keeps the one-sweep kernels), vectors off
@@ -27,8 +28,10 @@ def _option(gpu, value):
 
 @pytest.fixture
 def tile(gpu):
+    gpu.check(gpu.lib().lace_set_option(b"jacobi_tile", 2))
     yield lambda v: _option(gpu, v)
     _option(gpu, 1)
+    gpu.check(gpu.lib().lace_set_option(b"jacobi_tile", 1))
 
 
 @pytest.mark.parametrize("prec", PRECS)
@@ -75,3 +78,32 @@ def test_gaps_and_unaligned_vectors(gpu, orc, tile, prec):
         off = lambda d: C.c_void_p(d.ptr.value + es)  # noqa: E731
         gpu.check(gpu.lib().lace_parilu_apply(P.h, gpu.TRSV_JACOBI, 5, 0, off(dr), off(dz)))
         assert np.array_equal(dz.download()[1:], want, equal_nan=True)
+
+
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("dims,least", [
+    # sweeps from which boxes are taken, by (F64, F32, 16 bits)
+    ((20, 9, 17), (2, 2, 2)), ((64, 24, 1), (2, 2, 2)), ((29, 57, 1), (2, 2, 2)),
+    ((17, 25, 13), (2, 2, 2)), ((63, 64, 65), (2, 2, 2)), ((66, 64, 63), (2, 3, 3)), ((64, 66, 63), (2, 2, 2)),
+    ((101, 102, 103), (2, 3, 4))])
+def test_tiles_only_where_they_pay(gpu, orc, dims, least, prec):
+    """The launches of L's sweeps: one for up to five sweeps on boxes, else one
+    a sweep after the first; the results are those of one-sweep launches."""
+    A = _matrix(orc, dims)
+    P = gpu.ParILU(gpu.HostCSR.from_csr(A), getattr(gpu, "LACE_" + prec))
+    P.sweeps(2)
+    lib, r = gpu.lib(), np.random.default_rng(2).standard_normal(A.n_rows)
+    for k in (2, 3, 4, 5):
+        gpu.check(lib.lace_timing_enable(1))
+        gpu.check(lib.lace_timing_reset())
+        try:
+            z = P.apply(r, gpu.TRSV_JACOBI, k)
+            calls = gpu.timing_calls("trsv_jacobi_sweep_lower")
+        finally:
+            gpu.check(lib.lace_timing_enable(0))
+        assert calls == (1 if k >= least[min(PRECS.index(prec), 2)] else k - 1), k
+        _option(gpu, 0)
+        try:
+            assert np.array_equal(P.apply(r, gpu.TRSV_JACOBI, k), z), k
+        finally:
+            _option(gpu, 1)
