@@ -163,22 +163,27 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream_sweep_kernel(
 // row, which precede it: those among the thread's positions and the four
 // before them (the previous lanes', shuffled in before any branch) come
 // from registers, only earlier ones (rows longer than the window, the
-// first lanes of a wave) from memory, in the same ascending order.  With
-// MATCH (patterns whose strict positions have matches of their own) the
-// block's positions and the 16 before them are in LDS, from where a row's own
-// values come; row j's values are gathered two matches at a time for all of a
-// thread's positions together, and registers are held to six blocks per CU
-// (one round of the chip up to 786000 positions): 91000-row mesh FP64 23.0 ->
-// 21.2 us, 148000-row mesh FP32 25.2 -> 21.4 us, of which 14 us are the
-// 70 MB it moves.
+// first lanes of a wave) from memory, in the same ascending order.
+//
+// Where strict positions have matches of their own (M: kFewMatches or
+// kMatches), kMatches keeps the block's positions and the 16 before them in
+// LDS, from where a row's own values come; row j's values are gathered two
+// matches at a time for all of a thread's positions together, and registers
+// are held to six blocks per CU (one round of the chip up to 786000
+// positions): 91000-row mesh FP64 23.0 -> 21.2 us, 148000-row mesh FP32 25.2 ->
+// 21.4 us, of which 14 us are the 70 MB it moves.  kFewMatches takes them from
+// memory one after another and is ahead where few positions have any
+// (match_kind).
 //
 // With 16-bit storage (TS not T) the new values are rounded to 16 bits
 // relative to their row's scale before they are stored and compared, as
 // parilu_round16_kernel rounds them: l_ij by rs[prow], u_ji by rs[pcol] of
 // its position (100 x 77 x 53 BF16: 21 us a sweep for the two launches, 13 us
 // in one; reset 34 -> 17 us).
-template <typename T, typename TS, bool STEP, bool MATCH, int P>
-__global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_kernel(
+enum { kNoMatches = 0, kFewMatches = 1, kMatches = 2 };
+
+template <typename T, typename TS, bool STEP, int M, int P>
+__global__ __launch_bounds__(kSweepBS, M == kMatches ? 6 : 1) void parilu_stream4_sweep_kernel(
     int np, const int* __restrict__ pmeta, const int* __restrict__ mptr,
     const int* __restrict__ mpairs, const T* __restrict__ AL, const T* __restrict__ AU,
     const T* __restrict__ VLin, const T* __restrict__ VUin, T* __restrict__ VLout,
@@ -186,6 +191,7 @@ __global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_
     const int* __restrict__ pcol, const float* __restrict__ rs) {
 #pragma clang fp contract(off)
   static_assert(P == 2 || P == 4, "two or four positions per thread");
+  constexpr bool MATCH = M == kMatches;
   constexpr int MB = 2;  // matches whose operands are loaded together
   constexpr int W = 4;  // positions of the window before the thread's first
   const int b = xcd_block(blockIdx.x, gridDim.x);
@@ -352,6 +358,13 @@ __global__ __launch_bounds__(kSweepBS, MATCH ? 6 : 1) void parilu_stream4_sweep_
         }
       } else {
         T sL = al[e], sU = au[e];
+        if (M == kFewMatches) {
+          for (int t = mptr[p]; t < mptr[p + 1]; t++) {
+            const int qa = mpairs[2 * t], qc = mpairs[2 * t + 1];
+            sL = sL - VLin[qa] * VUin[qc];
+            sU = sU - VLin[qc] * VUin[qa];
+          }
+        }
         if (MATCH) {
 #pragma unroll
           for (int k = 0; k < MB; k++)
@@ -912,6 +925,7 @@ static int build_pattern(const data_d_matrix* A, ParILU* P, ParILUUse use) {
       mptr[P->nnzL] = (int)(pairs.size() / 2);
       LACE_TRY(upload(P->pmeta, meta.data(), sizeof(int) * P->nnzL));
       P->strict_matches = !pairs.empty();
+      P->matches = pairs.size() / 2;
       if (P->strict_matches) {
         LACE_TRY(upload(P->mptr, mptr.data(), sizeof(int) * (P->nnzL + 1)));
         LACE_TRY(upload(P->mpairs, pairs.data(), sizeof(int) * pairs.size()));
@@ -1043,6 +1057,21 @@ static void launch_sym(ParILU* P, bool with_step, int in, int out, int nb) {
         P->uval[out].as<T>(), nullptr);
 }
 
+// How the streaming kernel takes the matches of P's strict positions.  In
+// FP64 staging them pays where there are many, or several rounds of blocks
+// (FP32 stages half as much and is ahead almost throughout).  Few -> staged,
+// FP64: meshes (1.3 matches a position) of 1331 rows 7.0 -> 7.5 us, 13800
+// (105000 positions) 7.8 -> 7.8, 33000 10.8 -> 9.8; diagonals 1, 30, 31 (0.67)
+// of 10^5 rows 6.1 -> 6.5, 10^6 43.2 -> 38.4; 1, 2 with gaps (0.13) of 3 10^5
+// 7.0 -> 7.7, 2 10^6 40.6 -> 36.8; the one loss seen past 2^20 positions is 1,
+// 1500, 1501 with gaps (0.33), 10^6 rows 33.5 -> 31.9 but 2 10^6 79 -> 85.
+template <typename T>
+static int match_kind(const ParILU* P) {
+  if (!P->strict_matches) return kNoMatches;
+  if (sizeof(T) == 4 || P->nnzL >= (1 << 20)) return kMatches;
+  return P->matches >= 1.2 * ((double)P->nnzL - P->n) && P->nnzL >= 100000 ? kMatches : kFewMatches;
+}
+
 template <typename T>
 static int sweep_t(ParILU* P, bool with_step) {
   const int in = P->cur, out = 1 - P->cur;
@@ -1056,7 +1085,8 @@ static int sweep_t(ParILU* P, bool with_step) {
     // array either way); two where strict positions have matches, whose
     // operands take the registers
     constexpr int PP = sizeof(T) == 8 ? 2 : 4;
-    const int nb = ceil_div(P->nnzL, kSweepBS * (P->strict_matches ? 2 : PP));
+    const int kind = match_kind<T>(P);
+    const int nb = ceil_div(P->nnzL, kSweepBS * (kind != kNoMatches ? 2 : PP));
     auto go = [&](auto kern) {
       tr.launch(kern, dim3(nb), dim3(kSweepBS), P->nnzL, P->pmeta.as<int>(), P->mptr.as<int>(),
                 P->mpairs.as<int>(), P->AL.as<T>(), P->AU.as<T>(), P->lval[in].as<T>(),
@@ -1065,13 +1095,20 @@ static int sweep_t(ParILU* P, bool with_step) {
     };
     const auto stored = [&](auto ts) {
       using TS = decltype(ts);
-      if (P->strict_matches) {
-        if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, true, 2>);
-        else go(parilu_stream4_sweep_kernel<T, TS, false, true, 2>);
-      } else {
-        if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, false, PP>);
-        else go(parilu_stream4_sweep_kernel<T, TS, false, false, PP>);
+      if (kind == kMatches) {
+        if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, kMatches, 2>);
+        else go(parilu_stream4_sweep_kernel<T, TS, false, kMatches, 2>);
+        return;
       }
+      if constexpr (sizeof(T) == 8) {
+        if (kind == kFewMatches) {
+          if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, kFewMatches, 2>);
+          else go(parilu_stream4_sweep_kernel<T, TS, false, kFewMatches, 2>);
+          return;
+        }
+      }
+      if (with_step) go(parilu_stream4_sweep_kernel<T, TS, true, kNoMatches, PP>);
+      else go(parilu_stream4_sweep_kernel<T, TS, false, kNoMatches, PP>);
     };
     if constexpr (sizeof(T) == 8) {
       stored(0.0);

@@ -222,6 +222,7 @@ struct ParILU {
   // (k < j) as index pairs, present only when some position has one
   DevBuf pmeta, mptr, mpairs;
   bool strict_matches = false;
+  size_t matches = 0;  // of all strict positions
 
   // Triangular solves.  lower: L (CSRL arrays, values lval[cur]).
   // upper: U in CSR (diagonal first), values gathered from the CSC buffer

@@ -2,7 +2,8 @@
 CSR product and Jacobi sweeps on blocks of rows (empty, short and long rows, a
 row longer than a block's entry capacity, sizes around a block and the chip's
 block count), and ParILU sweeps whose positions have none, up to four and more
-matches, in both step modes."""
+matches, taken from memory one after another or staged in LDS, in every factor
+storage and both step modes."""
 import numpy as np
 import pytest
 
@@ -34,6 +35,8 @@ def _pattern(orc, n, offs, keep, seed, long_row=False):
 WIDE = [1, 2, 3, 30, 31, 32, 33]
 CASES = [("tiny", 1, [], 1.0, False), ("pair", 2, [1], 1.0, False), ("block", 256, WIDE[:4], 0.6, False),
          ("over", 257, WIDE[:4], 0.6, False), ("ragged", 5003, WIDE, 0.4, False), ("full", 3001, WIDE, 1.0, False),
+         # FP64: matches staged in LDS, for their number and for the positions'
+         ("wide", 20001, WIDE, 1.0, False), ("rounds", 350001, [1, 2, 3], 1.0, False),
          ("long", 9001, [1, 40, 41], 0.7, True), ("many", 300001, [1, 500, 501, 502], 0.5, False)]
 
 
@@ -87,3 +90,27 @@ def test_row_blocks(gpu, orc, name, n, offs, keep, long_row, prec):
         assert np.array_equal(P.apply(x, gpu.TRSV_JACOBI, k), jacobi(Ur, jacobi(Lf, x, False, k), True, k)), k
         got = P.apply(x, gpu.TRSV_JACOBI, k, trans=1)
         assert np.array_equal(got, jacobi(Lt, jacobi(Uc, x, False, k), True, k)), k
+
+
+@pytest.mark.parametrize("prec", ["F64", "F32", "BF16", "F16"])
+@pytest.mark.parametrize("name", ["block", "over", "ragged", "full", "wide", "long"])
+def test_parilu_sweeps_with_matches(gpu, orc, name, prec):
+    """Every sweep's factors, bit for bit, in every storage (the 16-bit ones
+    round inside the sweep) and with and without the step, which sums up to
+    3 10^5 squares in FP64 in another order (at most that many roundings)."""
+    _, n, offs, keep, long_row = next(c for c in CASES if c[0] == name)
+    A = _pattern(orc, n, offs, keep, 5, long_row)
+    storage = prec.lower() if prec in ("BF16", "F16") else None
+    dt = np.float64 if prec == "F64" else np.float32
+    print(f"sweeps with matches: {name} {prec} n={n} nnz={A.nnz}", flush=True)
+    P = gpu.ParILU(gpu.HostCSR.from_csr(A), getattr(gpu, "LACE_" + prec))
+    st = orc.ParILUState(A, dtype=dt, storage=storage)
+    anorm = np.linalg.norm(A.val)
+    for k in range(4):
+        got = P.sweeps(1, want_step=k % 2 == 0)
+        step = st.sweep("jacobi") / anorm
+        (_, _, lv), (_, _, uv) = P.factors()
+        assert np.array_equal(lv.astype(dt), st.Lval), (k, "L")
+        assert np.array_equal(uv.astype(dt), st.Uval), (k, "U")
+        if k % 2 == 0:
+            assert abs(got - step) <= 3e5 * 2.3e-16 * step, (k, got, step)
