@@ -652,10 +652,14 @@ int lace_daxpby(size_t m, double a, const double *x, double b, const double *y, 
 int lace_block_panel_qr(int n, int r0, const double *W, double *Y, double *Tb, double *Rt,
                         int *passes);
 
-/* Kernel-shape options for tuning runs.  "stream_rows_per_thread" (1, 2 or
- * 4): rows each thread owns in the CSR-stream SpMV and Jacobi sweeps
- * (default: blocks of rows of about 2000 entries; Jacobi sweeps without the
- * off-diagonal form: 2 for FP32 values, 1 for FP64).  "jacobi_ell" (0 or 1, default
+/* Kernel-shape options for tuning runs.  "row_blocks" (0..2,
+ * default 1): SpMV and Jacobi sweeps on CSR forms of short rows run on blocks
+ * of rows of about 2000 entries where that is expected to be faster (0: never,
+ * 2: always; Jacobi sweeps without the off-diagonal form have no such
+ * kernel), else on the CSR-stream kernels.  "stream_rows_per_thread" (0, 1, 2
+ * or 4, default 0): rows each thread owns in those (0: 2 for FP32 values, 1
+ * for FP64); a value other than 0 takes them in place of blocks of rows.
+ * "jacobi_ell" (0 or 1, default
  * 1): Jacobi sweeps of ILU factors with short rows use the ELLPACK form of
  * the off-diagonal entries (0: the off-diagonal CSR-stream form).
  * "spmv_ell" (0 or 1, default 1): SpMV of a matrix with at most 8 entries

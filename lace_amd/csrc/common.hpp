@@ -61,6 +61,10 @@ int noalloc_setup(int device);
 int ring_setup();
 // Kernel-shape option set through lace_set_option (dflt when unset).
 int get_option(const char* name, int dflt);
+// Products and Jacobi sweeps on CSR forms: on blocks of rows (option "row_blocks"), or with a fixed number of
+// rows a thread for values of elem_size bytes ("stream_rows_per_thread").
+bool row_blocks();
+int stream_rows(size_t elem_size);
 
 // ---------------------------------------------------------------- memory
 // Host arrays in the reference convention (include/dense_types.h:430-450):

@@ -240,6 +240,16 @@ int get_option(const char* name, int dflt) {
   return it == g_options.end() ? dflt : it->second;
 }
 
+bool row_blocks() {
+  if (get_option("stream_rows_per_thread", 0) != 0) return false;
+  return get_option("row_blocks", 1) != 0;
+}
+
+int stream_rows(size_t elem_size) {
+  const int rows = get_option("stream_rows_per_thread", 0);
+  return rows != 0 ? rows : elem_size == 8 ? 1 : 2;
+}
+
 }  // namespace lace
 
 using namespace lace;
@@ -351,8 +361,8 @@ extern "C" int lace_set_option(const char* name, int value) {
   LACE_REQUIRE(name != nullptr, DEV_ERR_INVALID_PTR, "lace_set_option: null name");
   const std::string key(name);
   if (key == "stream_rows_per_thread") {
-    LACE_REQUIRE(value == 1 || value == 2 || value == 4, DEV_ERR_ILLEGAL_VALUE,
-                 "stream_rows_per_thread must be 1, 2 or 4 (have %d)", value);
+    LACE_REQUIRE(value == 0 || value == 1 || value == 2 || value == 4, DEV_ERR_ILLEGAL_VALUE,
+                 "stream_rows_per_thread must be 0, 1, 2 or 4 (have %d)", value);
   } else if (key == "jacobi_ell" || key == "spmv_ell" || key == "jacobi_dia" || key == "spmv_dia" ||
              key == "jacobi_fuse" || key == "jacobi_dia_vec" || key == "jacobi_pipe" ||
              key == "matlab_log" || key == "jacobi_dia16" || key == "inner_ortho" || key == "trsv_exact_tiles" ||
@@ -360,7 +370,7 @@ extern "C" int lace_set_option(const char* name, int value) {
     LACE_REQUIRE(value == 0 || value == 1, DEV_ERR_ILLEGAL_VALUE, "%s must be 0 or 1 (have %d)", name, value);
   } else if (key == "trsv_exact_wgs_per_cu") {
     LACE_REQUIRE(value >= 0 && value <= 16, DEV_ERR_ILLEGAL_VALUE, "%s must be 0..16 (have %d)", name, value);
-  } else if (key == "trsv_exact_ring" || key == "jacobi_march" || key == "jacobi_tile") {
+  } else if (key == "trsv_exact_ring" || key == "jacobi_march" || key == "jacobi_tile" || key == "row_blocks") {
     LACE_REQUIRE(value >= 0 && value <= 2, DEV_ERR_ILLEGAL_VALUE, "%s must be 0..2 (have %d)", name, value);
   } else if (key == "trsv_exact") {
     LACE_REQUIRE(value == 0 || value == 1, DEV_ERR_ILLEGAL_VALUE, "%s must be 0 or 1 (have %d)", name, value);

@@ -143,7 +143,8 @@ __global__ __launch_bounds__(kStreamThreads) void spmv_stream_kernel(
   }
 }
 
-// The same on short blocks of rows (block_row_sum), the default.  Ragged
+// The same on short blocks of rows (block_row_sum), the default where
+// row_blocks says so.  Ragged
 // meshes of about 14 entries a row, against blocks of 256 R rows: 13800 rows
 // FP64 7.2 -> 4.6 us, 212000 rows FP64 13.7 -> 11.3 us (3.6 TB/s) and FP32
 // 12.0 -> 7.0 us, 10^6 rows FP64 40.6 -> 33.1 us, 2 10^6 rows FP64 109 -> 87 us
@@ -319,14 +320,14 @@ static int launch_spmv(const DevCSR& A, const TX* x, TY* y, const TY* b, double 
   }
   if (A.n > 0 && A.nnz <= 16LL * A.n) {
     // short rows (at most 16 per row on average): the stream kernels
-    const int R = get_option("stream_rows_per_thread", 0);
-    if (R == 0) {
+    if (row_blocks()) {
       const int rpb = rows_per_block(A.n, A.nnz);
       spmv_rows_kernel<TV, TX, TY, MODE><<<ceil_div(A.n, rpb), 256, 0, stream()>>>(
           A.n, rpb, A.row.as<int>(), A.col.as<int>(), A.val.as<TV>(), x, y, b, alpha, beta);
       LACE_HIP(hipGetLastError());
       return DEV_SUCCESS;
     }
+    const int R = stream_rows(sizeof(TV));
     if (R == 1) launch_stream<TV, TX, TY, MODE, 1>(A, x, y, b, alpha, beta);
     else if (R == 4) launch_stream<TV, TX, TY, MODE, 4>(A, x, y, b, alpha, beta);
     else launch_stream<TV, TX, TY, MODE, 2>(A, x, y, b, alpha, beta);

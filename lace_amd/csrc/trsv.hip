@@ -1276,7 +1276,7 @@ __global__ void tri_diag_div_kernel(int n, const T* __restrict__ dval, const T* 
   if (i < n) y[i] = r[i] / dval[i];
 }
 
-// The same sweep on short blocks of rows (block_row_sum), the default; with
+// The same sweep on short blocks of rows (block_row_sum), the default where row_blocks says so; with
 // y2 and d2 given it also writes y2 = yout / d2, the first sweep of a following
 // solve.  Five sweeps of L and U on ragged meshes, against blocks of 256 R
 // rows: 1320 rows FP64 35 -> 25 us, 91000 rows FP64 43 -> 34 us, 148000 rows
@@ -1309,18 +1309,16 @@ static void launch_jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* 
       P.n, P.srow.as<int>(), P.scol.as<int>(), P.sval.as<T>(), P.dval.as<T>(), r, yin, yout);
 }
 
-static bool jacobi_rows() { return get_option("stream_rows_per_thread", 0) == 0; }
-
-// y2, d2: with jacobi_rows only.
+// y2, d2: with row_blocks only.
 template <typename T, bool UNIT>
 static void jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* yout, T* y2, const T* d2) {
-  if (jacobi_rows()) {
+  if (row_blocks()) {
     const int rpb = rows_per_block(P.n, P.snnz);
     tri_jacobi_rows_kernel<T, UNIT><<<ceil_div(P.n, rpb), 256, 0, stream()>>>(
         P.n, rpb, P.srow.as<int>(), P.scol.as<int>(), P.sval.as<T>(), P.dval.as<T>(), r, yin, yout, y2, d2);
     return;
   }
-  const int R = get_option("stream_rows_per_thread", 0);
+  const int R = stream_rows(sizeof(T));
   if (R == 1) launch_jacobi_strict<T, UNIT, 1>(P, r, yin, yout);
   else if (R == 4) launch_jacobi_strict<T, UNIT, 4>(P, r, yin, yout);
   else launch_jacobi_strict<T, UNIT, 2>(P, r, yin, yout);
@@ -1335,7 +1333,7 @@ static void launch_jacobi_stream(const TriPlan& P, const T* val, const T* r, con
 template <typename T, bool UPPER>
 static void jacobi_stream(const TriPlan& P, const T* val, const T* r, const T* yin, T* yout) {
   // measured at 128^3: two rows per thread for FP32 values, one for FP64
-  const int R = get_option("stream_rows_per_thread", sizeof(T) == 8 ? 1 : 2);
+  const int R = stream_rows(sizeof(T));
   if (R == 1) launch_jacobi_stream<T, UPPER, 1>(P, val, r, yin, yout);
   else if (R == 4) launch_jacobi_stream<T, UPPER, 4>(P, val, r, yin, yout);
   else launch_jacobi_stream<T, UPPER, 2>(P, val, r, yin, yout);
@@ -1507,7 +1505,7 @@ static int jacobi_sweep(const TriPlan& P, const T* val, const T* r, const T* yin
   if (!partial && yin && P.n > 0 && P.nnz <= 16LL * P.n) {
     const bool dia = strict && P.dia.nd > 0 && get_option("jacobi_dia", 1) != 0;
     const bool ell = !dia && strict && P.ew > 0 && get_option("jacobi_ell", 1) != 0;
-    const bool fuse = (dia || (strict && !ell && jacobi_rows())) && y2 && d2;
+    const bool fuse = (dia || (strict && !ell && row_blocks())) && y2 && d2;
     // 16-bit words of the diagonal form where the factors are stored in 16
     // bits (four rows per thread; it needs n % 4 == 0 and aligned vectors)
     const bool d16 = dia && sizeof(T) == 4 && P.dia16_fmt != LACE_F32 && P.dia16_src == (const void*)val &&

@@ -1,7 +1,7 @@
 """Kernels on general short-row patterns against the oracle, bit for bit: the
-CSR product and Jacobi sweeps on blocks of rows (empty, short and long rows, a
-row longer than a block's entry capacity, sizes around a block and the chip's
-block count), and ParILU sweeps whose positions have none, up to four and more
+CSR product and Jacobi sweeps on blocks of rows and with 1, 2 and 4 rows a
+thread (empty, short and long rows, a row longer than a block's entry capacity,
+sizes around a block and the chip's block count), and ParILU sweeps whose positions have none, up to four and more
 matches, taken from memory one after another or staged in LDS, in every factor
 storage and both step modes."""
 import numpy as np
@@ -40,6 +40,28 @@ CASES = [("tiny", 1, [], 1.0, False), ("pair", 2, [1], 1.0, False), ("block", 25
          ("long", 9001, [1, 40, 41], 0.7, True), ("many", 300001, [1, 500, 501, 502], 0.5, False)]
 
 
+# the kernels of a CSR form, and the default choice among them
+KERNELS = [(b"row_blocks", 2, 1), (b"row_blocks", 0, 1), (b"stream_rows_per_thread", 1, 0),
+           (b"stream_rows_per_thread", 2, 0), (b"stream_rows_per_thread", 4, 0), (b"row_blocks", 1, 1)]
+
+
+def _each_kernel(gpu, call):
+    for name, value, default in KERNELS:
+        gpu.check(gpu.lib().lace_set_option(name, value))
+        try:
+            yield (name, value), call()
+        finally:
+            gpu.check(gpu.lib().lace_set_option(name, default))
+
+
+def test_row_options(lace):
+    """Every choice can be taken back to the default; others are refused."""
+    lib = lace.lib()
+    for name, ok, bad in ((b"row_blocks", (0, 2, 1), (-1, 3)), (b"stream_rows_per_thread", (1, 2, 4, 0), (-1, 3, 5))):
+        assert all(lib.lace_set_option(name, v) == 0 for v in ok)
+        assert all(lib.lace_set_option(name, v) != 0 for v in bad)
+
+
 @pytest.mark.parametrize("prec", ["F64", "F32"])
 @pytest.mark.parametrize("name,n,offs,keep,long_row", CASES)
 def test_row_blocks(gpu, orc, name, n, offs, keep, long_row, prec):
@@ -50,7 +72,7 @@ def test_row_blocks(gpu, orc, name, n, offs, keep, long_row, prec):
     rng = np.random.default_rng(4)
     x = rng.standard_normal(n).astype(dt)
     if A.nnz <= 16 * n:
-        y = gpu.DevCSRMatrix(H, getattr(gpu, "LACE_" + prec)).spmv(x)
+        M = gpu.DevCSRMatrix(H, getattr(gpu, "LACE_" + prec))
         # each row summed in column order from zero, in the values' precision
         ri = A.rowidx()
         prod = (A.val.astype(dt) * x[A.col]).astype(dt)
@@ -59,7 +81,9 @@ def test_row_blocks(gpu, orc, name, n, offs, keep, long_row, prec):
         for q in range(int(np.diff(A.row).max())):
             has = at + q < A.row[1:]
             want[has] = want[has] + prod[(at + q)[has]]
-        assert len(ri) == A.nnz and np.array_equal(y, want)
+        assert len(ri) == A.nnz
+        for kernel, y in _each_kernel(gpu, lambda: M.spmv(x)):
+            assert np.array_equal(y, want), kernel
     P = gpu.ParILU(H, getattr(gpu, "LACE_" + prec))
     P.sweeps(3)
     st = orc.parilu(A, 3, dtype=dt)
@@ -87,9 +111,12 @@ def test_row_blocks(gpu, orc, name, n, offs, keep, long_row, prec):
         return y
 
     for k in (2, 5):
-        assert np.array_equal(P.apply(x, gpu.TRSV_JACOBI, k), jacobi(Ur, jacobi(Lf, x, False, k), True, k)), k
-        got = P.apply(x, gpu.TRSV_JACOBI, k, trans=1)
-        assert np.array_equal(got, jacobi(Lt, jacobi(Uc, x, False, k), True, k)), k
+        want = jacobi(Ur, jacobi(Lf, x, False, k), True, k)
+        for kernel, got in _each_kernel(gpu, lambda: P.apply(x, gpu.TRSV_JACOBI, k)):
+            assert np.array_equal(got, want), (kernel, k)
+        want = jacobi(Lt, jacobi(Uc, x, False, k), True, k)
+        for kernel, got in _each_kernel(gpu, lambda: P.apply(x, gpu.TRSV_JACOBI, k, trans=1)):
+            assert np.array_equal(got, want), (kernel, k)
 
 
 @pytest.mark.parametrize("prec", ["F64", "F32", "BF16", "F16"])
