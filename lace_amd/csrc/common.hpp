@@ -61,9 +61,10 @@ int noalloc_setup(int device);
 int ring_setup();
 // Kernel-shape option set through lace_set_option (dflt when unset).
 int get_option(const char* name, int dflt);
-// Products and Jacobi sweeps on CSR forms: on blocks of rows (option "row_blocks"), or with a fixed number of
+// Products and Jacobi sweeps of n rows with off off-diagonal entries on CSR
+// forms: on blocks of rows (option "row_blocks"), or with a fixed number of
 // rows a thread for values of elem_size bytes ("stream_rows_per_thread").
-bool row_blocks();
+bool row_blocks(int n, long off);
 int stream_rows(size_t elem_size);
 
 // ---------------------------------------------------------------- memory

@@ -320,7 +320,7 @@ static int launch_spmv(const DevCSR& A, const TX* x, TY* y, const TY* b, double 
   }
   if (A.n > 0 && A.nnz <= 16LL * A.n) {
     // short rows (at most 16 per row on average): the stream kernels
-    if (row_blocks()) {
+    if (row_blocks(A.n, A.nnz - A.n)) {
       const int rpb = rows_per_block(A.n, A.nnz);
       spmv_rows_kernel<TV, TX, TY, MODE><<<ceil_div(A.n, rpb), 256, 0, stream()>>>(
           A.n, rpb, A.row.as<int>(), A.col.as<int>(), A.val.as<TV>(), x, y, b, alpha, beta);

@@ -1312,7 +1312,7 @@ static void launch_jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* 
 // y2, d2: with row_blocks only.
 template <typename T, bool UNIT>
 static void jacobi_strict(const TriPlan& P, const T* r, const T* yin, T* yout, T* y2, const T* d2) {
-  if (row_blocks()) {
+  if (row_blocks(P.n, P.snnz)) {
     const int rpb = rows_per_block(P.n, P.snnz);
     tri_jacobi_rows_kernel<T, UNIT><<<ceil_div(P.n, rpb), 256, 0, stream()>>>(
         P.n, rpb, P.srow.as<int>(), P.scol.as<int>(), P.sval.as<T>(), P.dval.as<T>(), r, yin, yout, y2, d2);
@@ -1505,7 +1505,7 @@ static int jacobi_sweep(const TriPlan& P, const T* val, const T* r, const T* yin
   if (!partial && yin && P.n > 0 && P.nnz <= 16LL * P.n) {
     const bool dia = strict && P.dia.nd > 0 && get_option("jacobi_dia", 1) != 0;
     const bool ell = !dia && strict && P.ew > 0 && get_option("jacobi_ell", 1) != 0;
-    const bool fuse = (dia || (strict && !ell && row_blocks())) && y2 && d2;
+    const bool fuse = (dia || (strict && !ell && row_blocks(P.n, P.snnz))) && y2 && d2;
     // 16-bit words of the diagonal form where the factors are stored in 16
     // bits (four rows per thread; it needs n % 4 == 0 and aligned vectors)
     const bool d16 = dia && sizeof(T) == 4 && P.dia16_fmt != LACE_F32 && P.dia16_src == (const void*)val &&
