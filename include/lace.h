@@ -721,7 +721,9 @@ int lace_block_panel_qr(int n, int r0, const double *W, double *Y, double *Tb, d
  * to about 260000 rows whose levels are narrow run in level order on one
  * workgroup, the last rows of the solution in LDS, where that is expected
  * to be faster (and "trsv_exact_tiles" and "trsv_exact_rows" are at their
- * defaults; 2: wherever the form exists).  Either way the result is bit-identical.
+ * defaults; 2: wherever the form exists; a handle holds it where it is
+ * expected to be faster, or in every case if made while this is 2).  Either
+ * way the result is bit-identical.
  * "inner_ortho" (0 or 1, default 1): the inner GMRES of a nested solve
  * (inner_iters > 0) orthogonalises by classical Gram-Schmidt on an
  * unnormalised basis (1: two vector passes and one small launch per step)

@@ -2,6 +2,7 @@
 // Krylov translation units.
 #pragma once
 
+#include <future>
 #include <vector>
 
 #include "common.hpp"
@@ -40,6 +41,14 @@ struct Sentinel<float> {
 // i.  `sched` lists rows level by level; each level starts on a multiple of
 // 64 slots (padding slots hold -1) so that one wavefront never holds two
 // levels -- the sync-free kernel relies on it.
+// Host part of a plan's level-order form (TriPlan::ring_host).
+struct RingHost {
+  int chunks = 0;  // 0: no such form
+  int groups = 0, span = 0;
+  int all_groups = 0;
+  std::vector<int> form;
+};
+
 struct TriPlan {
   int n = 0, nnz = 0;
   bool upper = false;
@@ -115,32 +124,51 @@ struct TriPlan {
   // padding), rslot each row's slot, ridx the off-diagonal operands' places
   // in that order modulo 2^15, four to a group.  rspan is the farthest back
   // an operand lies, which decides whether the solution's last rows fit in
-  // LDS.  rval / rdiag hold the values gathered from rval_src (cleared by
-  // refresh_strict), rrhs and rsol the right-hand side and the solution in
-  // that order.
+  // LDS.  Behind them, for values of the plan's type, lie the values (rval)
+  // and the diagonal (rdiag) gathered from rval_src (cleared by
+  // refresh_strict), the right-hand side (rrhs) and the solution (rsol).
   int rchunks = 0;  // 0: no such form
   int rgroups = 0;  // groups of four a row takes at most
   int rspan = 0;
   size_t rslots = 0;
-  DevBuf rform;  // rdesc, rperm, rslot, each row's place in level order, ridx
+  DevBuf rform;  // rdesc, rperm, rslot, each row's place in level order, ridx, the values
   const unsigned* rdesc() const { return rform.as<unsigned>(); }
   int* rperm() const { return rform.as<int>() + 2 * (size_t)rchunks; }
   int* rslot() const { return rperm() + 64 * (size_t)rchunks; }
   int* rplace() const { return rslot() + (n + 1) / 2 * 2; }
   unsigned short* ridx() const { return reinterpret_cast<unsigned short*>(rplace() + (n + 1) / 2 * 2); }
+  template <typename T> T* rval() const { return reinterpret_cast<T*>(ridx() + rslots); }
+  template <typename T> T* rdiag() const { return rval<T>() + rslots; }
+  template <typename T> T* rrhs() const { return rdiag<T>() + 64 * (size_t)rchunks; }
+  template <typename T> T* rsol() const { return rrhs<T>() + 64 * (size_t)rchunks; }
   size_t rform_words() const { return 66 * (size_t)rchunks + 2 * (size_t)((n + 1) / 2 * 2); }  // before ridx
-  mutable DevBuf rval, rdiag, rrhs, rsol;
+  size_t rform_bytes(size_t elem_size) const {
+    return sizeof(int) * rform_words() + 2 * rslots + elem_size * (rslots + 192 * (size_t)rchunks);
+  }
   mutable const void* rval_src = nullptr;
   static constexpr unsigned kFormStrict = 1, kFormDiag = 2, kFormEll = 4, kFormDia = 8, kFormAll = 15;
   unsigned stale = 0;  // forms not yet gathered from strict_src
   size_t src_es = 0;   // element size of strict_src
-  // jacobi / exact: whether the forms of those solves are wanted; same: a
-  // plan of the same pattern and triangle, if there is one
-  int build(int n, const int* row, const int* col, bool upper, bool jacobi = true, bool exact = true,
-            const TriPlan* same = nullptr);
+  // Level sets of a pattern; ring: begin the level-order form too, whose host
+  // part is worked out beside the caller's own work (on a thread where that is
+  // worth one) and ended by end_ring.  row and col must stay until then, or
+  // until wait_ring.
+  std::vector<int> h_perm;  // until build
+  std::future<RingHost> ring_host;
+  void levels(int n, const int* row, const int* col, bool upper, bool ring);
+  // The rest of the plan.  jacobi / exact: whether the forms of those solves
+  // are wanted; same: a plan of the same pattern and triangle, whose level sets
+  // are taken (levels need not have been called), and whose level-order form
+  // is taken with copy_ring.
+  int build(const int* row, const int* col, bool jacobi, bool exact, const TriPlan* same = nullptr);
   int build_tiles(const int* row, const int* col, bool exact);
-  int build_ring(const int* row, const int* col, const int* perm, const int* lptr);
-  int copy_ring(const TriPlan& o);
+  // host: what must stay until the stream is synchronised
+  int end_ring(size_t elem_size, RingHost* host);
+  void wait_ring() {
+    if (ring_host.valid()) ring_host.wait();
+  }
+  bool ring_copied = false;
+  int copy_ring(const TriPlan& o, size_t elem_size);
   int refresh_strict(const void* val, size_t elem_size);
   int ensure_forms(unsigned forms);
   // 16-bit diagonal form (fmt BF16 or F16) from the value array strict_src,

@@ -26,30 +26,42 @@
 namespace lace {
 
 // ---------------------------------------------------------------- plans
-int TriPlan::build(int n_, const int* row_, const int* col_, bool upper_, bool jacobi, bool exact,
-                   const TriPlan* same) {
-  n = n_;
-  nnz = row_[n_];
-  upper = upper_;
-  std::vector<int> perm_h(n), lptr_h(n + 1);
-  nlev = lace_level_sets(n, row_, col_, upper ? 1 : 0, perm_h.data(), lptr_h.data());
-  h_lptr.assign(lptr_h.begin(), lptr_h.begin() + nlev + 1);
-  std::vector<int> sched_h;
-  sched_h.reserve(n + 64 * (size_t)nlev);
-  for (int l = 0; l < nlev; l++) {
-    for (int t = h_lptr[l]; t < h_lptr[l + 1]; t++) sched_h.push_back(perm_h[t]);
-    while (sched_h.size() % 64) sched_h.push_back(-1);
+static int duplicate(DevBuf& d, const DevBuf& o) {
+  LACE_TRY(d.alloc(o.bytes));
+  LACE_HIP(hipMemcpyAsync(d.p, o.p, o.bytes, hipMemcpyDeviceToDevice, stream()));
+  return DEV_SUCCESS;
+}
+
+int TriPlan::build(const int* row_, const int* col_, bool jacobi, bool exact, const TriPlan* same) {
+  if (same) {
+    n = same->n;
+    nnz = same->nnz;
+    upper = same->upper;
+    nlev = same->nlev;
+    nslots = same->nslots;
+    maxoff = same->maxoff;
+    h_lptr = same->h_lptr;
+    LACE_TRY(duplicate(row, same->row));
+    LACE_TRY(duplicate(col, same->col));
+    LACE_TRY(duplicate(perm, same->perm));
+    LACE_TRY(duplicate(lptr, same->lptr));
+    LACE_TRY(duplicate(sched, same->sched));
+  } else {
+    std::vector<int> sched_h;
+    sched_h.reserve(n + 64 * (size_t)nlev);
+    for (int l = 0; l < nlev; l++) {
+      for (int t = h_lptr[l]; t < h_lptr[l + 1]; t++) sched_h.push_back(h_perm[t]);
+      while (sched_h.size() % 64) sched_h.push_back(-1);
+    }
+    nslots = (int)sched_h.size();
+    LACE_TRY(upload(row, row_, sizeof(int) * (n + 1)));
+    LACE_TRY(upload(col, col_, sizeof(int) * std::max(nnz, 1)));
+    LACE_TRY(upload(perm, h_perm.data(), sizeof(int) * std::max(n, 1)));
+    LACE_TRY(upload(lptr, h_lptr.data(), sizeof(int) * (nlev + 1)));
+    LACE_TRY(upload(sched, sched_h.data(), sizeof(int) * std::max(nslots, 1)));
+    std::vector<int>().swap(h_perm);
   }
-  nslots = (int)sched_h.size();
-  LACE_TRY(upload(row, row_, sizeof(int) * (n + 1)));
-  LACE_TRY(upload(col, col_, sizeof(int) * std::max(nnz, 1)));
-  LACE_TRY(upload(perm, perm_h.data(), sizeof(int) * std::max(n, 1)));
-  LACE_TRY(upload(lptr, h_lptr.data(), sizeof(int) * (nlev + 1)));
-  LACE_TRY(upload(sched, sched_h.data(), sizeof(int) * std::max(nslots, 1)));
   strict_src = nullptr;
-  maxoff = 0;
-  for (int i = 0; i < n; i++) maxoff = std::max(maxoff, row_[i + 1] - row_[i] - 1);
-  if (exact) LACE_TRY(same ? copy_ring(*same) : build_ring(row_, col_, perm_h.data(), lptr_h.data()));
   if (!jacobi) return build_tiles(row_, col_, exact);
   // off-diagonal form: every entry but the row's diagonal slot (first for
   // upper, last for lower), in row order
@@ -1736,39 +1748,54 @@ template int tri_solve_jacobi<float>(const TriPlan&, const float*, const float*,
 
 // ---------------------------------------------------------------- ParILU solves
 int ParILU::build_trsv(ParILUUse use) {
-  LACE_TRY(lower.build(n, h_lrow.data(), h_lcol.data(), false, use.jacobi, use.exact));
-  lower.unit_diag = true;  // CSRL with the unit diagonal (never updated by sweeps)
-  if (use.trans) LACE_TRY(lowerT.build(n, h_ucp.data(), h_uri.data(), false, use.jacobi, use.exact, sym ? &lower : nullptr));
-  // U in CSR: transpose of the CSC arrays; map CSR slot -> CSC slot.
-  {
-    std::vector<int> r(n + 1, 0), c(nnzU), map(nnzU);
-    for (int p = 0; p < nnzU; p++) r[h_uri[p] + 1]++;
+  // the plans' level orders are worked out from these arrays meanwhile
+  std::vector<int> ur, uc, ltr, ltc, umap, ltmap;
+  struct Wait {
+    ParILU* P;
+    ~Wait() {
+      for (TriPlan* t : {&P->lower, &P->upper, &P->lowerT, &P->upperT}) t->wait_ring();
+    }
+  } wait{this};
+  // CSR of the transpose of (ptr, idx): map CSR slot ->
+  // slot of the arrays given
+  const auto transpose = [this](const std::vector<int>& ptr, const std::vector<int>& idx, int m, std::vector<int>& r,
+                                std::vector<int>& c, std::vector<int>& map) {
+    r.assign(n + 1, 0);
+    c.resize(m);
+    map.resize(m);
+    for (int p = 0; p < m; p++) r[idx[p] + 1]++;
     for (int i = 0; i < n; i++) r[i + 1] += r[i];
     std::vector<int> fill(r.begin(), r.end() - 1);
     for (int j = 0; j < n; j++)
-      for (int p = h_ucp[j]; p < h_ucp[j + 1]; p++) {
-        int q = fill[h_uri[p]]++;
+      for (int p = ptr[j]; p < ptr[j + 1]; p++) {
+        const int q = fill[idx[p]]++;
         c[q] = j;
         map[q] = p;
       }
-    LACE_TRY(upper.build(n, r.data(), c.data(), true, use.jacobi, use.exact));
-    LACE_TRY(upload(u_csr_from_csc, map.data(), sizeof(int) * nnzU));
-  }
-  // L^T in CSR (diagonal first): transpose of L's CSR arrays.
+  };
+  // L; U in CSR, the transpose of the CSC arrays; U^T; L^T in CSR (diagonal
+  // first), the transpose of L's CSR arrays.  On a symmetric pattern U^T takes
+  // L's level sets and L^T takes U's, and their level orders with the first
+  // transposed exact solve.
+  lower.levels(n, h_lrow.data(), h_lcol.data(), false, use.exact);
+  transpose(h_ucp, h_uri, nnzU, ur, uc, umap);
+  upper.levels(n, ur.data(), uc.data(), true, use.exact);
   if (use.trans) {
-    std::vector<int> r(n + 1, 0), c(nnzL), map(nnzL);
-    for (int p = 0; p < nnzL; p++) r[h_lcol[p] + 1]++;
-    for (int i = 0; i < n; i++) r[i + 1] += r[i];
-    std::vector<int> fill(r.begin(), r.end() - 1);
-    for (int i = 0; i < n; i++)
-      for (int p = h_lrow[i]; p < h_lrow[i + 1]; p++) {
-        int q = fill[h_lcol[p]]++;
-        c[q] = i;
-        map[q] = p;
-      }
-    LACE_TRY(upperT.build(n, r.data(), c.data(), true, use.jacobi, use.exact, sym ? &upper : nullptr));
+    transpose(h_lrow, h_lcol, nnzL, ltr, ltc, ltmap);
+    if (!sym) {
+      lowerT.levels(n, h_ucp.data(), h_uri.data(), false, use.exact);
+      upperT.levels(n, ltr.data(), ltc.data(), true, use.exact);
+    }
+  }
+  LACE_TRY(lower.build(h_lrow.data(), h_lcol.data(), use.jacobi, use.exact));
+  lower.unit_diag = true;  // CSRL with the unit diagonal (never updated by sweeps)
+  LACE_TRY(upper.build(ur.data(), uc.data(), use.jacobi, use.exact));
+  LACE_TRY(upload(u_csr_from_csc, umap.data(), sizeof(int) * nnzU));
+  if (use.trans) {
+    LACE_TRY(lowerT.build(h_ucp.data(), h_uri.data(), use.jacobi, use.exact, sym ? &lower : nullptr));
+    LACE_TRY(upperT.build(ltr.data(), ltc.data(), use.jacobi, use.exact, sym ? &upper : nullptr));
     upperT.unit_diag = true;
-    LACE_TRY(upload(l_t_from_csr, map.data(), sizeof(int) * nnzL));
+    LACE_TRY(upload(l_t_from_csr, ltmap.data(), sizeof(int) * nnzL));
   }
   const size_t es = elem_size();
   LACE_TRY(uval_csr.alloc(es * nnzU));
@@ -1777,6 +1804,10 @@ int ParILU::build_trsv(ParILUUse use) {
   LACE_TRY(work2.alloc(es * n));
   LACE_TRY(syncfree_err.alloc(sizeof(int) * 4));
   LACE_HIP(hipMemsetAsync(syncfree_err.p, 0, sizeof(int) * 4, stream()));
+  RingHost host[4];
+  int k = 0;
+  for (TriPlan* t : {&lower, &upper, &lowerT, &upperT}) LACE_TRY(t->end_ring(es, &host[k++]));
+  LACE_HIP(hipStreamSynchronize(stream()));  // host is released on return
   csr_dirty = true;
   return DEV_SUCCESS;
 }
@@ -1837,6 +1868,10 @@ int ParILU::prepare(lace_trsv_kind_t kind, int trans, bool block, int sweeps) {
           nnzL, l_t_from_csr.as<int>(), lval[cur].as<float>(), lval_t.as<float>());
     LACE_HIP(hipGetLastError());
     lval_t_dirty = false;
+  }
+  if (kind == LACE_TRSV_LEVEL && trans && sym) {
+    if (!lowerT.ring_copied) LACE_TRY(lowerT.copy_ring(lower, elem_size()));
+    if (!upperT.ring_copied) LACE_TRY(upperT.copy_ring(upper, elem_size()));
   }
   if (kind == LACE_TRSV_JACOBI) {
     TriPlan& a = trans ? lowerT : lower;

@@ -14,6 +14,8 @@
 // by its remainder was slower than dividing (75 against 66 us on 64 x 64: the
 // exponent test and its branch cost what the division's steps do).
 #include <algorithm>
+#include <new>
+#include <system_error>
 
 #include "common.hpp"
 #include "device.hpp"
@@ -96,24 +98,23 @@ static void ring_levels(int n, const int* row, const int* col, bool upper, int r
   }
 }
 
-int TriPlan::build_ring(const int* row_, const int* col_, const int* perm_h, const int* lptr_h) {
-  rchunks = 0;
-  rval_src = nullptr;
-  if (n < 1 || maxoff > 16 || nlev >= (1 << kRingLevelBits) - 1) return DEV_SUCCESS;
+static RingHost ring_plan(int n, const int* row, const int* col, bool upper, int maxoff, int nlev,
+                          const std::vector<int>& perm, std::vector<int> lptr) {
+  RingHost h;
   // whole rounds of two chunks a wave, the last ones empty
   const auto padded = [](long chunks) { return (chunks + 2 * kRingWaves - 1) / (2 * kRingWaves) * (2 * kRingWaves); };
-  if (padded(((long)n + 63) / 64) > kRingDescs) return DEV_SUCCESS;
-  const auto len = [&](int i) { return row_[i + 1] - row_[i] - 1; };
-  std::vector<int> lev(n), pos(n), order(n), lptr(nlev + 1), at;
+  if (n < 1 || maxoff > 16 || nlev >= (1 << kRingLevelBits) - 1 || padded(((long)n + 63) / 64) > kRingDescs) return h;
+  const auto len = [&](int i) { return row[i + 1] - row[i] - 1; };
+  std::vector<int> lev(n), pos(n), order(n), at;
   for (int l = 0; l < nlev; l++)
-    for (int t = lptr_h[l]; t < lptr_h[l + 1]; t++) lev[perm_h[t]] = l;
+    for (int t = lptr[l]; t < lptr[l + 1]; t++) lev[perm[t]] = l;
   int span = 0, widest = 0;
   for (int pass = 0;; pass++) {
     // rows by level and, in a level, by falling length, so that a chunk's
     // rows need the same number of slots
     at.assign((size_t)nlev * 17 + 1, 0);
     for (int i = 0; i < n; i++) {
-      if (len(i) < 0) return DEV_SUCCESS;
+      if (len(i) < 0) return h;
       at[(size_t)lev[i] * 17 + 16 - len(i) + 1]++;
     }
     for (size_t q = 1; q < at.size(); q++) at[q] += at[q - 1];
@@ -123,10 +124,10 @@ int TriPlan::build_ring(const int* row_, const int* col_, const int* perm_h, con
     span = widest = 0;
     for (int l = 0; l < nlev; l++) widest = std::max(widest, lptr[l + 1] - lptr[l]);
     for (int i = 0; i < n; i++)
-      for (int k = row_[i]; k < row_[i + 1]; k++) {
-        const int j = col_[k];
+      for (int k = row[i]; k < row[i + 1]; k++) {
+        const int j = col[k];
         if (j == i) continue;
-        if (lev[j] >= lev[i]) return DEV_SUCCESS;  // not a triangular factor: no such form
+        if (lev[j] >= lev[i]) return h;  // not a triangular factor: no such form
         // a solved row must still be in the ring while its reader's level writes
         span = std::max(span, lptr[lev[i] + 1] - pos[j]);
       }
@@ -134,17 +135,16 @@ int TriPlan::build_ring(const int* row_, const int* col_, const int* perm_h, con
     // readers (ragged 47 x 45 x 46 mesh: 31 operands of 672 thousand more
     // than 16384 rows back, 31482 at most; 8139 after)
     if (span <= ring_rows<double>() || pass == 1) break;
-    ring_levels(n, row_, col_, upper, std::max(1, ring_rows<double>() / (2 * widest)), lev);
+    ring_levels(n, row, col, upper, std::max(1, ring_rows<double>() / (2 * widest)), lev);
   }
-  if (span > ring_rows<float>()) return DEV_SUCCESS;
+  if (span > ring_rows<float>()) return h;
   long chunks = 0;
   for (int l = 0; l < nlev; l++) chunks += (lptr[l + 1] - lptr[l] + 63) / 64;
   const int all = (int)padded(chunks);
-  if (all > kRingDescs) return DEV_SUCCESS;
-  rchunks = all;
-  std::vector<int> form(rform_words(), -1);
-  uint2* desc = reinterpret_cast<uint2*>(form.data());
-  int* rp = form.data() + 2 * (size_t)all;
+  if (all > kRingDescs) return h;
+  h.form.assign(66 * (size_t)all + 2 * (size_t)((n + 1) / 2 * 2), -1);
+  uint2* desc = reinterpret_cast<uint2*>(h.form.data());
+  int* rp = h.form.data() + 2 * (size_t)all;
   int* slot = rp + 64 * (size_t)all;
   std::copy(pos.begin(), pos.end(), slot + (n + 1) / 2 * 2);
   int c = 0, groups = 0, gmax = 1;
@@ -165,19 +165,91 @@ int TriPlan::build_ring(const int* row_, const int* col_, const int* perm_h, con
     desc[c].x = (unsigned)groups << 11;
     desc[c].y = (unsigned)(nlev - 1) << 15;
   }
+  h.chunks = all;
+  h.groups = gmax;
+  h.all_groups = groups;
+  h.span = span;
+  return h;
+}
+
+// One workgroup against the whole chip: 0.19 us a level plus the entries at
+// 100 GB/s and 8 ns a chunk, against 0.5 us a level in boxes of a 2-D grid,
+// 0.65 us in boxes of a 3-D grid and 1.6 us in runs of consecutive rows.
+// Measured on either side for L and U (FP64): 32^3 85 against 118 us (here),
+// 48^3 227 against 182 us (there), 400 x 300 397 against 704 us (here).
+static double ring_us(int nlev, size_t slots, int chunks, size_t elem_size) {
+  return 0.19 * nlev + 1e-5 * ((double)slots * (elem_size + 2.0) + 192.0 * chunks * elem_size) + 0.008 * chunks;
+}
+static double chip_us(const TriPlan& P) {
+  return P.nlev * (P.tile_dims[0] == 0 ? 1.6 : P.tile_dims[2] > 1 ? 0.65 : 0.5);
+}
+static bool ring_pays(const TriPlan& P, size_t elem_size) {
+  return ring_us(P.nlev, P.rslots, P.rchunks, elem_size) < 0.9 * chip_us(P);
+}
+
+// Making a handle of a 91000-row mesh took 42.7 ms without level orders, 47.5
+// with their host parts in line, and takes 40.8 with them beside the other
+// forms (and the transposes' level sets copied).  A thread costs about what
+// planning 8000 rows takes; without one the host part runs in end_ring.
+void TriPlan::levels(int n_, const int* row_, const int* col_, bool upper_, bool ring) {
+  n = n_;
+  nnz = row_[n_];
+  upper = upper_;
+  h_perm.resize(n);
+  std::vector<int> lptr_h(n + 1);
+  nlev = lace_level_sets(n, row_, col_, upper ? 1 : 0, h_perm.data(), lptr_h.data());
+  h_lptr.assign(lptr_h.begin(), lptr_h.begin() + nlev + 1);
+  maxoff = 0;
+  for (int i = 0; i < n; i++) maxoff = std::max(maxoff, row_[i + 1] - row_[i] - 1);
+  rval_src = nullptr;
+  rchunks = 0;
+  // not where it could not pay even with full chunks, against the slowest
+  // blocks of the persistent kernel
+  if (!ring || n == 0 ||
+      (get_option("trsv_exact_ring", 1) != 2 && ring_us(nlev, std::max(0, nnz - n), ceil_div(n, 64), 4) >= 1.44 * nlev))
+    return;
+  auto task = [n = n, row_, col_, upper = upper, maxoff = maxoff, nlev = nlev, perm = h_perm, lptr = h_lptr] {
+    return ring_plan(n, row_, col_, upper, maxoff, nlev, perm, lptr);
+  };
+  if (n >= 8000) {
+    try {
+      ring_host = std::async(std::launch::async, task);
+      return;
+    } catch (const std::system_error&) {  // no thread to be had
+    }
+  }
+  ring_host = std::async(std::launch::deferred, std::move(task));
+}
+
+// The form is kept where it is expected to pay (option "trsv_exact_ring" 2:
+// wherever there is one).  Without memory for it a plan has none, and its exact
+// solves run the persistent kernel, which needs no more than the factor.
+int TriPlan::end_ring(size_t elem_size, RingHost* host) {
+  if (!ring_host.valid()) return DEV_SUCCESS;
+  RingHost& h = *host;
+  try {
+    h = ring_host.get();
+  } catch (const std::bad_alloc&) {
+    return DEV_SUCCESS;
+  }
+  if (h.chunks == 0) return DEV_SUCCESS;
   // one more group: where a chunk without operands points
-  rslots = ((size_t)groups + 1) * 256;
-  const size_t words = rform_words();
-  rchunks = 0;  // until the form is there
-  LACE_TRY(rform.alloc(sizeof(int) * words + sizeof(uint16_t) * rslots));
-  LACE_HIP(hipMemcpyAsync(rform.p, form.data(), sizeof(int) * words, hipMemcpyHostToDevice, stream()));
-  LACE_HIP(hipStreamSynchronize(stream()));  // form is released on return
-  rchunks = all;
-  ring_index_kernel<<<all + 1, 64, 0, stream()>>>(all, reinterpret_cast<const uint2*>(rdesc()), rperm(),
-                                                  row.as<int>(), col.as<int>(), rplace(), upper, groups, ridx());
+  rslots = ((size_t)h.all_groups + 1) * 256;
+  rgroups = h.groups;
+  rspan = h.span;
+  rchunks = h.chunks;
+  const bool fits = rspan <= kRingBytes / (int)elem_size;
+  if (!fits || (get_option("trsv_exact_ring", 1) != 2 && !ring_pays(*this, elem_size)) ||
+      rform.alloc(rform_bytes(elem_size)) != DEV_SUCCESS) {
+    (void)hipGetLastError();
+    rchunks = 0;
+    return DEV_SUCCESS;
+  }
+  LACE_HIP(hipMemcpyAsync(rform.p, h.form.data(), sizeof(int) * h.form.size(), hipMemcpyHostToDevice, stream()));
+  ring_index_kernel<<<rchunks + 1, 64, 0, stream()>>>(rchunks, reinterpret_cast<const uint2*>(rdesc()), rperm(),
+                                                      row.as<int>(), col.as<int>(), rplace(), upper, h.all_groups,
+                                                      ridx());
   LACE_HIP(hipGetLastError());
-  rgroups = gmax;
-  rspan = span;
   return DEV_SUCCESS;
 }
 
@@ -196,16 +268,21 @@ __global__ __launch_bounds__(256) void ring_move_kernel(int m, const int* __rest
 
 // The form of a plan with the same pattern and triangle (symmetric patterns:
 // U^T has L's, L^T has U's).
-int TriPlan::copy_ring(const TriPlan& o) {
+int TriPlan::copy_ring(const TriPlan& o, size_t elem_size) {
+  ring_copied = true;
   rval_src = nullptr;
-  rchunks = 0;
-  if (o.rchunks == 0) return DEV_SUCCESS;
-  LACE_TRY(rform.alloc(o.rform.bytes));
-  LACE_HIP(hipMemcpyAsync(rform.p, o.rform.p, o.rform.bytes, hipMemcpyDeviceToDevice, stream()));
+  rchunks = o.rchunks;
+  if (rchunks == 0) return DEV_SUCCESS;
   rslots = o.rslots;
   rgroups = o.rgroups;
   rspan = o.rspan;
-  rchunks = o.rchunks;
+  if (rform.alloc(rform_bytes(elem_size)) != DEV_SUCCESS) {
+    (void)hipGetLastError();
+    rchunks = 0;
+    return DEV_SUCCESS;
+  }
+  LACE_HIP(hipMemcpyAsync(rform.p, o.rform.p, sizeof(int) * rform_words() + 2 * rslots, hipMemcpyDeviceToDevice,
+                          stream()));
   return DEV_SUCCESS;
 }
 
@@ -350,22 +427,13 @@ __global__ __launch_bounds__(W * 64) void tri_ring_kernel(int nlev, int nchunks,
   reach(nlev);
 }
 
-// One workgroup against the whole chip: 0.19 us a level plus the entries at
-// 100 GB/s and 8 ns a chunk, against 0.5 us a level in boxes of a 2-D grid,
-// 0.65 us in boxes of a 3-D grid and 1.6 us in runs of consecutive rows.
-// Measured on either side for L and U (FP64): 32^3 85 against 118 us (here),
-// 48^3 227 against 182 us (there), 400 x 300 397 against 704 us (here).
 template <typename T>
 bool ring_ready(const TriPlan& P) {
   const int ring = get_option("trsv_exact_ring", 1);
   if (ring == 0 || P.rchunks == 0 || P.rspan > ring_rows<T>()) return false;
-  if (ring == 2) return true;
-  const double bytes = (double)P.rslots * (sizeof(T) + 2.0) + 64.0 * P.rchunks * 3.0 * sizeof(T);
-  const double one = 0.19 * P.nlev + 1e-5 * bytes + 0.008 * P.rchunks;
-  const double chip = P.nlev * (P.tile_dims[0] == 0 ? 1.6 : P.tile_dims[2] > 1 ? 0.65 : 0.5);
   // options that shape the persistent kernel ask for that kernel
-  return one < 0.9 * chip && get_option("trsv_exact_tiles", 1) != 0 &&
-         get_option("trsv_exact_rows", 512) == 512;
+  return ring == 2 || (ring_pays(P, sizeof(T)) && get_option("trsv_exact_tiles", 1) != 0 &&
+                       get_option("trsv_exact_rows", 512) == 512);
 }
 
 // The kernels' LDS is past what a launch may ask for by itself: allowed for
@@ -399,7 +467,7 @@ template <typename T, int NG, int W, bool DIRECT>
 static int ring_launch(const TriPlan& P, const T* rhs, T* out) {
   const size_t lds = kRingBytes + 16 + sizeof(uint2) * P.rchunks;
   tri_ring_kernel<T, NG, W, DIRECT><<<1, W * 64, lds, stream()>>>(
-      P.nlev, P.rchunks, reinterpret_cast<const uint2*>(P.rdesc()), P.rval.as<T>(), reinterpret_cast<const ushort4*>(P.ridx()), rhs, P.rdiag.as<T>(),
+      P.nlev, P.rchunks, reinterpret_cast<const uint2*>(P.rdesc()), P.rval<T>(), reinterpret_cast<const ushort4*>(P.ridx()), rhs, P.rdiag<T>(),
       P.rperm(), out);
   LACE_HIP(hipGetLastError());
   return DEV_SUCCESS;
@@ -429,17 +497,13 @@ static int ring_solve(const TriPlan& P, const T* rhs, T* out) {
 // mesh (290) 152 against 155 us, 200 x 200 (800) 254 against 209 us.
 static bool ring_direct(const TriPlan& P) { return P.rchunks <= 320; }
 
-// The plan's buffers and the values of val in chunk order.
+// The values of val in chunk order.
 template <typename T>
 static int ring_values(const TriPlan& P, const T* val) {
   if (P.rval_src == (const void*)val) return DEV_SUCCESS;
-  const size_t rows = (size_t)P.rchunks * 64;
-  if (P.rval.bytes < sizeof(T) * P.rslots) LACE_TRY(P.rval.alloc(sizeof(T) * P.rslots));
-  for (DevBuf* b : {&P.rdiag, &P.rrhs, &P.rsol})
-    if (b->bytes < sizeof(T) * rows) LACE_TRY(b->alloc(sizeof(T) * rows));
   ring_gather_kernel<T><<<P.rchunks + 1, 64, 0, stream()>>>(P.rchunks, reinterpret_cast<const uint2*>(P.rdesc()), P.rperm(),
                                                             P.row.as<int>(), P.upper, P.rslots, val,
-                                                            P.rval.as<T>(), P.rdiag.as<T>());
+                                                            P.rval<T>(), P.rdiag<T>());
   LACE_HIP(hipGetLastError());
   P.rval_src = val;
   return DEV_SUCCESS;
@@ -457,20 +521,20 @@ int tri_solve_ring(const TriPlan& P, const T* val, const T* r, T* y) {
   LACE_REQUIRE((const void*)r != (const void*)y, DEV_ERR_ILLEGAL_VALUE, "exact solve needs distinct r and y");
   LACE_TRY(ring_values<T>(P, val));
   if (ring_direct(P)) return ring_solve<T, true>(P, r, y);
-  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm(), nullptr, r, P.rrhs.as<T>()));
-  LACE_TRY((ring_solve<T, false>(P, P.rrhs.as<T>(), P.rsol.as<T>())));
-  return ring_move<T>(P.n, P.rslot(), nullptr, P.rsol.as<T>(), y);
+  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm(), nullptr, r, P.rrhs<T>()));
+  LACE_TRY((ring_solve<T, false>(P, P.rrhs<T>(), P.rsol<T>())));
+  return ring_move<T>(P.n, P.rslot(), nullptr, P.rsol<T>(), y);
 }
 
 template <typename T>
 int tri_solve_ring2(const TriPlan& P, const T* val, const TriPlan& Q, const T* val2, const T* r, T* y) {
   LACE_TRY(ring_values<T>(P, val));
   LACE_TRY(ring_values<T>(Q, val2));
-  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm(), nullptr, r, P.rrhs.as<T>()));
-  LACE_TRY((ring_solve<T, false>(P, P.rrhs.as<T>(), P.rsol.as<T>())));
-  LACE_TRY(ring_move<T>(Q.rchunks * 64, Q.rperm(), P.rslot(), P.rsol.as<T>(), Q.rrhs.as<T>()));
-  LACE_TRY((ring_solve<T, false>(Q, Q.rrhs.as<T>(), Q.rsol.as<T>())));
-  return ring_move<T>(Q.n, Q.rslot(), nullptr, Q.rsol.as<T>(), y);
+  LACE_TRY(ring_move<T>(P.rchunks * 64, P.rperm(), nullptr, r, P.rrhs<T>()));
+  LACE_TRY((ring_solve<T, false>(P, P.rrhs<T>(), P.rsol<T>())));
+  LACE_TRY(ring_move<T>(Q.rchunks * 64, Q.rperm(), P.rslot(), P.rsol<T>(), Q.rrhs<T>()));
+  LACE_TRY((ring_solve<T, false>(Q, Q.rrhs<T>(), Q.rsol<T>())));
+  return ring_move<T>(Q.n, Q.rslot(), nullptr, Q.rsol<T>(), y);
 }
 
 template <typename T>
