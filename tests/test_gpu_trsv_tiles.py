@@ -9,7 +9,9 @@ consecutive-row blocks -- for L and U, for the transposed solves, after the
 factor values change, with 256-row blocks, and on grids whose sides are not
 multiples of the box.  Patterns that only look like a grid (offsets 1, nx,
 nx*ny with entries that wrap round a grid line) and general patterns keep
-consecutive-row blocks."""
+consecutive-row blocks.  The one-workgroup solve, which takes most of these
+sizes by default (option "trsv_exact_ring"), is off here, and compared with
+substitution beside them where it has a form."""
 import numpy as np
 import pytest
 
@@ -53,13 +55,22 @@ def _opt(gpu, name, value):
     gpu.check(gpu.lib().lace_set_option(name.encode(), value))
 
 
+@pytest.fixture(autouse=True)
+def persistent(gpu):
+    _opt(gpu, "trsv_exact_ring", 0)
+    yield
+    _opt(gpu, "trsv_exact_ring", 1)
+
+
 @pytest.mark.parametrize("name", ["convdiff", "laplace2d", "wrap", "trefethen20", "tiny", "chain"])
 @pytest.mark.parametrize("prec", ["f64", "f32"])
 def test_exact_solve_box_order(gpu, orc, name, prec):
     A = _problem(orc, name)
     lp, dt = (gpu.LACE_F64, np.float64) if prec == "f64" else (gpu.LACE_F32, np.float32)
     print(f"box order: {name} {prec} n={A.n_rows}", flush=True)
+    _opt(gpu, "trsv_exact_ring", 2)
     P = gpu.ParILU(gpu.HostCSR.from_csr(A), lp)
+    _opt(gpu, "trsv_exact_ring", 0)
     for w in range(4):
         assert P.tiles(w) == WANT[name], (w, P.tiles(w))
     r = np.random.default_rng(11).standard_normal(A.n_rows).astype(dt)
@@ -87,6 +98,12 @@ def test_exact_solve_box_order(gpu, orc, name, prec):
             assert np.array_equal(P.apply(r, gpu.TRSV_LEVEL), got)
         finally:
             _opt(gpu, "trsv_exact_rows", 512)
+        _opt(gpu, "trsv_exact_ring", 2)
+        try:
+            assert np.array_equal(P.apply(r, gpu.TRSV_LEVEL), want)
+            assert np.array_equal(P.apply(r, gpu.TRSV_LEVEL, trans=1), got_t)
+        finally:
+            _opt(gpu, "trsv_exact_ring", 0)
 
 
 def test_exact_solve_box_order_solver(gpu, orc):
