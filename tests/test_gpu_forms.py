@@ -1,9 +1,9 @@
 """Storage forms of the products and Jacobi sweeps.  The diagonal (DIA),
 ELLPACK and CSR forms give bit-identical results (the oracle's, in FP64);
 which forms a matrix gets follows its pattern.  The Jacobi sweeps on the
-diagonal form run pipelined (all sweeps of a factor in one launch) or one
-launch per sweep with 16 bytes of rows or one row per thread, also
-bit-identical."""
+diagonal form run pipelined (all sweeps of a factor in one launch), several to
+a launch on boxes of a full grid, or one launch per sweep with 16 bytes of rows
+or one row per thread, also bit-identical."""
 import ctypes as C
 import os
 
@@ -28,6 +28,7 @@ def forms(gpu):
         set_forms(kind, "dia")
     gpu.check(gpu.lib().lace_set_option(b"jacobi_fuse", 1))
     gpu.check(gpu.lib().lace_set_option(b"jacobi_dia_vec", 1))
+    gpu.check(gpu.lib().lace_set_option(b"jacobi_tile", 1))
     gpu.check(gpu.lib().lace_set_option(b"jacobi_pipe", 0))
 
 
@@ -99,13 +100,15 @@ def test_jacobi_forms_bitexact(gpu, orc, forms, name, prec):
             for fuse in (1, 0):
                 gpu.check(gpu.lib().lace_set_option(b"jacobi_fuse", fuse))
                 # diagonal form: all sweeps of a factor in one pipelined
-                # launch, or a launch per sweep with a 16-byte word of rows
-                # per thread or one row
-                for pipe, vec in (((1, 1), (0, 1), (0, 0)) if form == "dia" else ((0, 1),)):
+                # launch, on boxes (full grids), or a launch per sweep with a
+                # 16-byte word of rows per thread or one row
+                for pipe, vec, tile in (((1, 1, 0), (0, 1, 2), (0, 1, 0), (0, 0, 0)) if form == "dia"
+                                        else ((0, 1, 1),)):
                     gpu.check(gpu.lib().lace_set_option(b"jacobi_pipe", pipe))
                     gpu.check(gpu.lib().lace_set_option(b"jacobi_dia_vec", vec))
+                    gpu.check(gpu.lib().lace_set_option(b"jacobi_tile", tile))
                     got = P.apply(r, gpu.TRSV_JACOBI, sweeps=sweeps)
-                    assert np.array_equal(got, ref), (form, fuse, pipe, vec, sweeps)
+                    assert np.array_equal(got, ref), (form, fuse, pipe, vec, tile, sweeps)
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32"])

@@ -64,8 +64,8 @@ def test_parilu16_bitexact(gpu, orc, storage, name, variant):
 @pytest.mark.parametrize("storage", ["bf16", "f16"])
 @pytest.mark.parametrize("name", ["convdiff16", "scaled_rows", "nonsym"])
 def test_parilu16_solves_bitexact(gpu, orc, storage, name):
-    """Jacobi-5 (the diagonal form reads the 16-bit words on the stencil)
-    and exact solves with the 16-bit factors equal the oracle's FP32 solves
+    """Jacobi-5 (the diagonal form reads the 16-bit words on the stencil, on
+    boxes of the grid and in one-sweep launches) and exact solves with the 16-bit factors equal the oracle's FP32 solves
     on the oracle's factors, and the Jacobi result is the same with the FP32
     copy of the diagonal form."""
     A = _problem(orc, name)
@@ -76,8 +76,13 @@ def test_parilu16_solves_bitexact(gpu, orc, storage, name):
     r = np.random.default_rng(7).standard_normal(A.n_rows).astype(np.float32)
     y = orc.trsv_jacobi(Lf, r, False, 5, dtype=np.float32)
     want = orc.trsv_jacobi(Uf, y, True, 5, dtype=np.float32)
-    got = P.apply(r, kind=gpu.TRSV_JACOBI, sweeps=5)
-    assert np.array_equal(got, want)
+    for tile in (2, 0, 1):
+        gpu.check(gpu.lib().lace_set_option(b"jacobi_tile", tile))
+        try:
+            got = P.apply(r, kind=gpu.TRSV_JACOBI, sweeps=5)
+        finally:
+            gpu.check(gpu.lib().lace_set_option(b"jacobi_tile", 1))
+        assert np.array_equal(got, want), tile
     gpu.check(gpu.lib().lace_set_option(b"jacobi_dia16", 0))
     try:
         got32 = P.apply(r, kind=gpu.TRSV_JACOBI, sweeps=5)
