@@ -170,10 +170,11 @@ __global__ __launch_bounds__(kSweepBS) void parilu_stream_sweep_kernel(
 // LDS, from where a row's own values come; row j's values are gathered two
 // matches at a time for all of a thread's positions together, and registers
 // are held to six blocks per CU (one round of the chip up to 786000
-// positions): 91000-row mesh FP64 23.0 -> 21.2 us, 148000-row mesh FP32 25.2 ->
-// 21.4 us, of which 14 us are the 70 MB it moves.  kFewMatches takes them from
-// memory one after another and is ahead where few positions have any
-// (match_kind).
+// positions): 91000-row mesh FP64 23.0 -> 21.2 us for 47 MB of streams (6 us at
+// the rate of a copy; the rest are the waits of the chain mptr, mpairs, row j's
+// values, which come from cache), 149000-row mesh FP32 25.2 -> 21.4 us (49 MB).
+// kFewMatches takes them from memory one after another and is ahead where few
+// positions have any (match_kind).
 //
 // With 16-bit storage (TS not T) the new values are rounded to 16 bits
 // relative to their row's scale before they are stored and compared, as

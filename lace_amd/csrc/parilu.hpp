@@ -83,8 +83,10 @@ struct TriPlan {
   DiaForm dia;
   // For factors stored in 16 bits (BF16 or F16): the diagonal form's values
   // and the diagonal as 16-bit words relative to each row's power-of-two
-  // scale, and that scale's exponent per row; refreshed from the FP32 forms
-  // by refresh_dia16 (the Jacobi sweeps use them when called with dia16_src).
+  // scale, and that scale's exponent per row; encoded by refresh_dia16 from
+  // strict_src, the factor's own values, whether or not the FP32 forms are
+  // gathered (the Jacobi sweeps use them when called with dia16_src; solves on
+  // boxes that read nothing else leave the FP32 forms stale).
   lace_prec_t dia16_fmt = LACE_F32;
   DevBuf dia16, dexp, dval16;
   const void* dia16_src = nullptr;
