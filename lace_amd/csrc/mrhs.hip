@@ -776,6 +776,8 @@ static bool jacobi32_march_applies(const TriPlan& P, const float* val, int K) {
                      P.n <= (1 << 29) && P.grid[0] < 4096 && P.grid[1] < 4096 && get_option("jacobi_dia", 1) != 0 &&
                      get_option("jacobi_pair", 1) != 0;
   if (!there || march != 1) return there && march == 2;
+  // (nothing under 80000 rows was ahead: no shape is worked out for those)
+  if (K == 1 || P.n < (1 << 16)) return false;
   const int shortest = K / march_launches(K), longest = ceil_div(K, march_launches(K));
   return march_pays(march_shape(P, longest)) && (shortest == longest || march_pays(march_shape(P, shortest)));
 }
