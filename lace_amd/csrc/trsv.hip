@@ -1749,17 +1749,16 @@ template int tri_solve_jacobi<float>(const TriPlan&, const float*, const float*,
 // ---------------------------------------------------------------- ParILU solves
 int ParILU::build_trsv(ParILUUse use) {
   // the plans' level orders are worked out from these arrays meanwhile
-  std::vector<int> ur, uc, ltr, ltc, umap, ltmap;
+  std::vector<int> ur, uc, ltr, ltc, map;
   struct Wait {
     ParILU* P;
     ~Wait() {
       for (TriPlan* t : {&P->lower, &P->upper, &P->lowerT, &P->upperT}) t->wait_ring();
     }
   } wait{this};
-  // CSR of the transpose of (ptr, idx): map CSR slot ->
-  // slot of the arrays given
-  const auto transpose = [this](const std::vector<int>& ptr, const std::vector<int>& idx, int m, std::vector<int>& r,
-                                std::vector<int>& c, std::vector<int>& map) {
+  // CSR of the transpose of (ptr, idx); map: each CSR slot's place in idx
+  const auto transpose = [&](const std::vector<int>& ptr, const std::vector<int>& idx, int m, std::vector<int>& r,
+                             std::vector<int>& c) {
     r.assign(n + 1, 0);
     c.resize(m);
     map.resize(m);
@@ -1778,10 +1777,12 @@ int ParILU::build_trsv(ParILUUse use) {
   // L's level sets and L^T takes U's, and their level orders with the first
   // transposed exact solve.
   lower.levels(n, h_lrow.data(), h_lcol.data(), false, use.exact);
-  transpose(h_ucp, h_uri, nnzU, ur, uc, umap);
+  transpose(h_ucp, h_uri, nnzU, ur, uc);
   upper.levels(n, ur.data(), uc.data(), true, use.exact);
+  LACE_TRY(upload(u_csr_from_csc, map.data(), sizeof(int) * nnzU));
   if (use.trans) {
-    transpose(h_lrow, h_lcol, nnzL, ltr, ltc, ltmap);
+    transpose(h_lrow, h_lcol, nnzL, ltr, ltc);
+    LACE_TRY(upload(l_t_from_csr, map.data(), sizeof(int) * nnzL));
     if (!sym) {
       lowerT.levels(n, h_ucp.data(), h_uri.data(), false, use.exact);
       upperT.levels(n, ltr.data(), ltc.data(), true, use.exact);
@@ -1790,12 +1791,10 @@ int ParILU::build_trsv(ParILUUse use) {
   LACE_TRY(lower.build(h_lrow.data(), h_lcol.data(), use.jacobi, use.exact));
   lower.unit_diag = true;  // CSRL with the unit diagonal (never updated by sweeps)
   LACE_TRY(upper.build(ur.data(), uc.data(), use.jacobi, use.exact));
-  LACE_TRY(upload(u_csr_from_csc, umap.data(), sizeof(int) * nnzU));
   if (use.trans) {
     LACE_TRY(lowerT.build(h_ucp.data(), h_uri.data(), use.jacobi, use.exact, sym ? &lower : nullptr));
     LACE_TRY(upperT.build(ltr.data(), ltc.data(), use.jacobi, use.exact, sym ? &upper : nullptr));
     upperT.unit_diag = true;
-    LACE_TRY(upload(l_t_from_csr, ltmap.data(), sizeof(int) * nnzL));
   }
   const size_t es = elem_size();
   LACE_TRY(uval_csr.alloc(es * nnzU));
